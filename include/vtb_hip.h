@@ -350,8 +350,10 @@ int vtb_hip_matmul_q6_k(VtbHipCtx *ctx, VtbHipBuf *out_buf, VtbHipBuf *w_buf, si
  * are exact and sums f32 (results agree with the CPU path to ~1e-6 of
  * sum |W||x|).  k a multiple of the block size and at most 32768 (the
  * reference's MAX_K: error 5 above it); weights 4-byte aligned, below 2 GiB.
- * The context keeps a scratch of 4*Bp*k + Bp*k/4 + 4*Bp bytes (Bp = B
- * rounded up to 128), grown on demand.  vtb_hip_matmul_batched_* run synchronously. */
+ * The context keeps a scratch of about 4*Bp*k + Bp*k/8 + 4*Bp bytes (Bp = B
+ * rounded up to 32, above 32 to 64; k to 256) and, once a call has too few
+ * tokens and rows to fill the chip and splits k, 2 * CUs * 64 KiB of partials;
+ * both grow on demand.  vtb_hip_matmul_batched_* run synchronously. */
 void vtb_hip_segment_matmul_batched_q8_0(VtbHipSeg *seg, VtbHipBuf *out_buf, VtbHipBuf *w_buf, size_t w_offset,
                                          VtbHipBuf *acts_buf, size_t m, size_t k, size_t B);
 void vtb_hip_segment_matmul_batched_q4_k(VtbHipSeg *seg, VtbHipBuf *out_buf, VtbHipBuf *w_buf, size_t w_offset,

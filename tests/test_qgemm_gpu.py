@@ -143,3 +143,21 @@ def test_shared_prepass_blocks_match_single_calls(ctx, kind):
             seg.matmul_batched(kind, o, wb, off, xb, m, k, B)
     for g, s1, m in zip(grouped, single, ms):
         assert np.array_equal(ctx.download(g, np.float32, B * m), ctx.download(s1, np.float32, B * m))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("m,k,B", [(255, 256, 32), (257, 768, 33), (256, 1280, 64), (300, 2816, 65), (20, 256, 2047),
+                                   (20, 512, 2049)])
+def test_tile_and_split_edges(ctx, orc, kind, m, k, B):
+    # one 32-token tile and the first 64-token one, row blocks of 256 and one
+    # row either side, one block of k per split and uneven splits (11 blocks),
+    # the pre-pass's forms for few and many tokens
+    batched_case(ctx, orc, kind, m, k, B, seed=m + k + B)
+
+
+@pytest.mark.parametrize("k", [32, 96, 288, 1056])
+@pytest.mark.parametrize("B", [3, 70])
+def test_q8_0_odd_block_counts(ctx, orc, k, B):
+    # k ending inside a 64-column chunk, and inside a block of 256 (rows then
+    # start at 2-byte alignment); the last split shorter than the others
+    batched_case(ctx, orc, "q8_0", 130, k, B, seed=k + B)

@@ -209,33 +209,47 @@ static_assert(offsetof(GemvArgs, w1) == 56 && offsetof(GemvArgs, w2) == 80 && of
 // Batched-matmul activation pre-pass (vtb_xsplit).
 struct XSplitArgs {
   const float* x;      // [B][k]
-  uint16_t* planes;    // [2][Bp][k] f16 bits: h1, h2 of x * 2^e
-  float* sums;         // [Bp][k / 16]: sum of each 16-column group of x * 2^e
-  float* inv_scale;    // [Bp]: 2^-e of each token
-  int B;
-  int Bp;              // B rounded up to the token tile; rows >= B are zero
+  uint16_t* planes;    // f16 bits of h1, h2 of x * 2^e in fragment order, whole 32-token tiles
+  uint16_t* sums;      // [tiles][ceil(k / 256)][64][8]: sums of 32 columns of x * 2^(e - 5) as two f16 pieces
+  float* inv_scale;    // [32 tiles]: 2^-e of each token
+  int B;               // tokens past B are written as zeros
   int k;
-  int pad;
 };
-static_assert(sizeof(XSplitArgs) == 48 && offsetof(XSplitArgs, B) == 32, "XSplitArgs layout");
+static_assert(sizeof(XSplitArgs) == 40 && offsetof(XSplitArgs, B) == 32, "XSplitArgs layout");
 
 // Batched quantised matmul (vtb_qgemm_*).
 struct QGemmArgs {
   const uint8_t* w;          // m rows of row_bytes
-  const uint16_t* planes;    // [2][Bp][k] f16 bits from vtb_xsplit
-  const float* sums;         // [Bp][k / 16] (of x * 2^e)
-  const float* inv_scale;    // [Bp]: 2^-e
+  const uint16_t* planes;    // from vtb_xsplit
+  const uint16_t* sums;
+  const float* inv_scale;
   float* out;                // [B][m]
+  float* part;               // [n_split][n_tb][n_rb][64 or 32 tokens][256 rows] when n_split > 1
   unsigned w_bytes;          // m * row_bytes rounded up to a multiple of 4
   int m;
   int k;
   int B;
-  int Bp;
   int row_bytes;
-  int n_rb;                  // row blocks of 128
-  int n_tb;                  // token blocks of 128
+  int n_rb;                  // row blocks of 256
+  int n_tb;                  // token blocks of 64 (vtb_qgemm_*_t64) or 32 (_t32)
+  int n_split;               // workgroups along k,
+  int split_blocks;          // each of this many 256-column blocks
+  int pad;
 };
-static_assert(sizeof(QGemmArgs) == 72 && offsetof(QGemmArgs, w_bytes) == 40, "QGemmArgs layout");
+static_assert(sizeof(QGemmArgs) == 88 && offsetof(QGemmArgs, w_bytes) == 48, "QGemmArgs layout");
+
+// The partials of a split matmul added into out (vtb_qgemm_reduce).
+struct QReduceArgs {
+  const float* part;         // [n_split][n_tb][n_rb][tile_tokens][256]
+  float* out;                // [B][m]
+  int m;
+  int B;
+  int n_rb;
+  int n_tb;
+  int tile_tokens;
+  int n_split;
+};
+static_assert(sizeof(QReduceArgs) == 40 && offsetof(QReduceArgs, m) == 16, "QReduceArgs layout");
 
 // Row-wise rmsnorm (vtb_rmsnorm_f32); one workgroup per row (gridDim.x rows).
 struct RmsNormArgs {

@@ -31,6 +31,7 @@ using vtb::FillArgs;
 using vtb::GemvArgs;
 using vtb::PrefillArgs;
 using vtb::QGemmArgs;
+using vtb::QReduceArgs;
 using vtb::RmsNormArgs;
 using vtb::RopeRowsArgs;
 using vtb::KvtArgs;
@@ -94,11 +95,11 @@ struct VtbHipCtx {
   hipFunction_t f_copy = nullptr;
   hipFunction_t f_fill = nullptr;
   hipFunction_t f_gemv[kNumQuant][kNumGemvR] = {};  // vtb_gemv_<kind>_r<1|2|4>
-  hipFunction_t f_xsplit = nullptr;
+  hipFunction_t f_xsplit = nullptr, f_xsplit_1 = nullptr, f_qgemm_reduce = nullptr;
   hipModule_t mod_layer = nullptr;  // rmsnorm, swiglu, gelu_approx, residual_add
   hipFunction_t f_rmsnorm = nullptr, f_swiglu = nullptr, f_gelu = nullptr, f_resadd = nullptr, f_addnorm = nullptr;
   hipFunction_t f_rope_rows = nullptr;
-  hipFunction_t f_qgemm[kNumQuant] = {};  // vtb_qgemm_<kind>
+  hipFunction_t f_qgemm[kNumQuant][2] = {};  // vtb_qgemm_<kind>_t<32|64>
   // Split-K workspace and arrival counters (counters are zero between launches).
   void* ws = nullptr;
   size_t ws_bytes = 0;
@@ -112,10 +113,12 @@ struct VtbHipCtx {
   // (bf16 caches), the per-tile statistics and exponents.
   void* pf = nullptr;
   size_t pf_bytes = 0;
-  // Batched-matmul activation scratch: three bf16 planes [3][Bp][k] and the
-  // 16-column sums [Bp][k/16], written by vtb_xsplit.
+  // Batched-matmul activation scratch, written by vtb_xsplit (qgemm_scratch).
   void* qg = nullptr;
   size_t qg_bytes = 0;
+  // Partials of matmuls split along k (qgemm_part_bytes).
+  void* qp = nullptr;
+  size_t qp_bytes = 0;
   // RoPE inverse-frequency tables 1/base^(2j/d) on the device, one per
   // (base, head_dim) seen; the host copy stays alive for the async upload.
   struct RopeTable {
@@ -762,19 +765,38 @@ int launch_gemv(VtbHipCtx* ctx, int qk, float* out, const void* w, const float* 
   return launch_gemv_blocks(ctx, qk, 1, outs, ws, ms, x, k);
 }
 
-// Batched-matmul scratch for B tokens of width k: two bf16 planes
-// [2][Bp][k], the 16-column sums [Bp][k/16] and the inverse scales [Bp],
-// Bp = B rounded up to 128.
-size_t qgemm_scratch_bytes(size_t B, size_t k) {
-  const size_t Bp = (B + 127) / 128 * 128;
-  return 2 * Bp * k * 2 + Bp * (k / 16) * 4 + Bp * 4;
+// Batched-matmul scratch for B tokens of width k, in whole tiles: tokens Bp (B
+// rounded up to 32 up to one tile, else to 64), the two f16 pieces in
+// fragment order (k rounded up to 64-column chunks), the sub-block sums (two
+// f16 per 32 columns, k rounded up to 256) and the inverse scales.
+struct QgemmScratch {
+  size_t tokens, sums, inv, bytes;
+};
+QgemmScratch qgemm_scratch(size_t B, size_t k) {
+  QgemmScratch q;
+  q.tokens = B <= 32 ? 32 : (B + 63) / 64 * 64;
+  q.sums = q.tokens * ((k + 63) / 64 * 64) * 4;
+  q.inv = q.sums + q.tokens * ((k + 255) / 256) * 32;
+  q.bytes = q.inv + q.tokens * 4;
+  return q;
 }
+constexpr size_t kQgRows = 256;  // rows of a workgroup
+// Partials of the matmuls whose k range is split: one tile of f32 per
+// workgroup, at most two workgroups per CU.
+size_t qgemm_part_bytes(VtbHipCtx* ctx) { return 2 * (size_t)std::max(ctx->cu_count, 1) * 64 * kQgRows * sizeof(float); }
 
 // Batched quantised matmul launcher: out[B][m] = acts[B][k] . W^T.  The
 // pre-pass scales each token by a power of two and splits it into two f16
-// planes, 16-column sums and the token's inverse scale in the
-// context's scratch (grown on demand, after the stream drains); the GEMM
-// then runs one workgroup per 128 tokens x 128 rows.
+// pieces, the sub-block sums and the token's inverse scale in the context's
+// scratch (grown on demand, after the stream drains); its one-token workgroups
+// run while eight-token ones would not fill the CUs once.  The GEMM then runs
+// one workgroup per token tile, 256 rows and share of k: k is split while
+// two workgroups per CU (what its registers allow) are not there otherwise,
+// in whole blocks of 256 columns, and vtb_qgemm_reduce adds the partials.
+// (Q4_K 1024 x 4096, 2048 tokens, 128 workgroups unsplit: 164 us with the former
+// 128 x 128 tiles, 72 split by four; 4096 x 4096, 33 tokens, 16 workgroups
+// unsplit: 151 and 23.)  Partials are tiles of 64 KiB, so n_split n_rb n_tb
+// <= 2 CUs bounds them whatever m and B.
 // Up to three weight matrices of one format over the same activations share
 // one pre-pass (the Q/K/V or gate/up projections of a prefill layer).
 int launch_qgemm_blocks(VtbHipCtx* ctx, int qk, int nblk, float* const outs[], const void* const ws[],
@@ -794,14 +816,12 @@ int launch_qgemm_blocks(VtbHipCtx* ctx, int qk, int nblk, float* const outs[], c
     if ((uintptr_t)ws[b] % 4 != 0) return set_err(ctx, VTB_HIP_EINVAL, "matmul_batched: weights not 4-byte aligned");
   }
   if (!aligned16(acts)) return set_err(ctx, VTB_HIP_EINVAL, "matmul_batched: activations not 16-byte aligned");
-  const size_t Bp = (B + 127) / 128 * 128;
-  const size_t planes_bytes = 2 * Bp * k * 2, sums_bytes = Bp * (k / 16) * 4;
-  int rc0 = ensure_scratch(ctx, &ctx->qg, &ctx->qg_bytes, qgemm_scratch_bytes(B, k),
-                           "hipMalloc(batched matmul scratch)");
-  if (rc0) return rc0;
+  const QgemmScratch qs = qgemm_scratch(B, k);
+  int rc = ensure_scratch(ctx, &ctx->qg, &ctx->qg_bytes, qs.bytes, "hipMalloc(batched matmul scratch)");
+  if (rc) return rc;
   uint16_t* planes = (uint16_t*)ctx->qg;
-  float* sums = (float*)((char*)ctx->qg + planes_bytes);
-  float* inv_scale = (float*)((char*)ctx->qg + planes_bytes + sums_bytes);
+  uint16_t* sums = (uint16_t*)((char*)ctx->qg + qs.sums);
+  float* inv_scale = (float*)((char*)ctx->qg + qs.inv);
   XSplitArgs xa;
   memset(&xa, 0, sizeof xa);
   xa.x = acts;
@@ -809,11 +829,24 @@ int launch_qgemm_blocks(VtbHipCtx* ctx, int qk, int nblk, float* const outs[], c
   xa.sums = sums;
   xa.inv_scale = inv_scale;
   xa.B = (int)B;
-  xa.Bp = (int)Bp;
   xa.k = (int)k;
-  int rc = launch(ctx, ctx->f_xsplit, (unsigned)Bp, 1, 1, 256, &xa);
+  const bool few = qs.tokens < 8 * (size_t)std::max(ctx->cu_count, 1);
+  rc = launch(ctx, few ? ctx->f_xsplit_1 : ctx->f_xsplit, (unsigned)(few ? qs.tokens : qs.tokens / 8), 1, 1, 256, &xa);
   if (rc) return rc;
+  const size_t tile = qs.tokens <= 32 ? 32 : 64;
+  const size_t n_tb = qs.tokens / tile, n256 = (k + 255) / 256;
   for (int b = 0; b < nblk; ++b) {
+    const size_t n_rb = (ms[b] + kQgRows - 1) / kQgRows;
+    if (n_rb * n_tb > 0x3fffffff) return set_err(ctx, VTB_HIP_EUNSUPPORTED, "matmul_batched: too many tokens or rows");
+    size_t n_split = std::max((size_t)1, 2 * (size_t)std::max(ctx->cu_count, 1) / (n_rb * n_tb));
+    n_split = (size_t)env_int("VTB_QGEMM_SPLIT", (int)n_split);
+    n_split = std::min(n_split, n256);
+    const size_t split_blocks = (n256 + n_split - 1) / n_split;
+    n_split = (n256 + split_blocks - 1) / split_blocks;
+    if (n_split > 1) {
+      rc = ensure_scratch(ctx, &ctx->qp, &ctx->qp_bytes, qgemm_part_bytes(ctx), "hipMalloc(batched matmul partials)");
+      if (rc) return rc;
+    }
     QGemmArgs a;
     memset(&a, 0, sizeof a);
     a.w = (const uint8_t*)ws[b];
@@ -821,18 +854,34 @@ int launch_qgemm_blocks(VtbHipCtx* ctx, int qk, int nblk, float* const outs[], c
     a.sums = sums;
     a.inv_scale = inv_scale;
     a.out = outs[b];
+    a.part = (float*)ctx->qp;
     // Rounded up to whole dwords: the last 2-byte-aligned field can end two
     // bytes into one (see launch_gemv).
     a.w_bytes = (unsigned)((ms[b] * row_bytes + 3) & ~(size_t)3);
     a.m = (int)ms[b];
     a.k = (int)k;
     a.B = (int)B;
-    a.Bp = (int)Bp;
     a.row_bytes = (int)row_bytes;
-    a.n_rb = (int)((ms[b] + 127) / 128);
-    a.n_tb = (int)(Bp / 128);
-    rc = launch(ctx, ctx->f_qgemm[qk], (unsigned)(a.n_rb * a.n_tb), 1, 1, 256, &a);
+    a.n_rb = (int)n_rb;
+    a.n_tb = (int)n_tb;
+    a.n_split = (int)n_split;
+    a.split_blocks = (int)split_blocks;
+    rc = launch(ctx, ctx->f_qgemm[qk][tile == 64], (unsigned)(n_rb * n_tb * n_split), 1, 1, 256, &a);
     if (rc) return rc;
+    if (n_split > 1) {
+      QReduceArgs r;
+      memset(&r, 0, sizeof r);
+      r.part = a.part;
+      r.out = outs[b];
+      r.m = a.m;
+      r.B = a.B;
+      r.n_rb = a.n_rb;
+      r.n_tb = a.n_tb;
+      r.tile_tokens = (int)tile;
+      r.n_split = a.n_split;
+      rc = launch(ctx, ctx->f_qgemm_reduce, (unsigned)n_rb, (unsigned)((B + 3) / 4), 1, 256, &r);
+      if (rc) return rc;
+    }
   }
   return VTB_HIP_OK;
 }
@@ -994,6 +1043,8 @@ extern "C" VtbHipCtx* vtb_hip_init(void) {
       ok = hipModuleGetFunction(&ctx->f_gemv[qk][ri], ctx->mod_gemv, name) == hipSuccess;
     }
   ok = ok && hipModuleGetFunction(&ctx->f_xsplit, ctx->mod_qgemm, "vtb_xsplit") == hipSuccess;
+  ok = ok && hipModuleGetFunction(&ctx->f_xsplit_1, ctx->mod_qgemm, "vtb_xsplit_1") == hipSuccess;
+  ok = ok && hipModuleGetFunction(&ctx->f_qgemm_reduce, ctx->mod_qgemm, "vtb_qgemm_reduce") == hipSuccess;
   ok = ok && hipModuleGetFunction(&ctx->f_rmsnorm, ctx->mod_layer, "vtb_rmsnorm_f32") == hipSuccess;
   ok = ok && hipModuleGetFunction(&ctx->f_swiglu, ctx->mod_layer, "vtb_swiglu_f32") == hipSuccess;
   ok = ok && hipModuleGetFunction(&ctx->f_gelu, ctx->mod_layer, "vtb_gelu_approx_f32") == hipSuccess;
@@ -1001,8 +1052,10 @@ extern "C" VtbHipCtx* vtb_hip_init(void) {
   ok = ok && hipModuleGetFunction(&ctx->f_addnorm, ctx->mod_layer, "vtb_add_rmsnorm_f32") == hipSuccess;
   ok = ok && hipModuleGetFunction(&ctx->f_rope_rows, ctx->mod_layer, "vtb_rope_rows_f32") == hipSuccess;
   for (int qk = 0; ok && qk < kNumQuant; ++qk) {
-    snprintf(name, sizeof name, "vtb_qgemm_%s", kQuantNames[qk]);
-    ok = hipModuleGetFunction(&ctx->f_qgemm[qk], ctx->mod_qgemm, name) == hipSuccess;
+    for (int t = 0; ok && t < 2; ++t) {
+      snprintf(name, sizeof name, "vtb_qgemm_%s_t%d", kQuantNames[qk], 32 << t);
+      ok = hipModuleGetFunction(&ctx->f_qgemm[qk][t], ctx->mod_qgemm, name) == hipSuccess;
+    }
   }
   (void)hipGetLastError();  // absent optional kernels are not an error for the caller
   if (!ok) {
@@ -1040,6 +1093,7 @@ extern "C" void vtb_hip_destroy(VtbHipCtx* ctx) {
   if (ctx->counters) (void)hipFree(ctx->counters);
   if (ctx->pf) (void)hipFree(ctx->pf);
   if (ctx->qg) (void)hipFree(ctx->qg);
+  if (ctx->qp) (void)hipFree(ctx->qp);
   for (auto& t : ctx->rope_tables) (void)hipFree(t.dev);
   if (ctx->mod_decode) (void)hipModuleUnload(ctx->mod_decode);
   if (ctx->mod_prefill) (void)hipModuleUnload(ctx->mod_prefill);
@@ -1826,8 +1880,10 @@ extern "C" int vtb_hip_reserve(VtbHipCtx* ctx, const VtbHipAttnConfig* cfg, int 
   }
   if (max_matmul_k > 0 && max_batch > 0) {
     if (max_matmul_k > 32768) return set_err(ctx, VTB_HIP_EUNSUPPORTED, "reserve: matmul k above 32768");
-    rc = ensure_scratch(ctx, &ctx->qg, &ctx->qg_bytes, qgemm_scratch_bytes(max_batch, max_matmul_k),
+    rc = ensure_scratch(ctx, &ctx->qg, &ctx->qg_bytes, qgemm_scratch(max_batch, max_matmul_k).bytes,
                         "hipMalloc(batched matmul scratch)");
+    if (rc) return rc;
+    rc = ensure_scratch(ctx, &ctx->qp, &ctx->qp_bytes, qgemm_part_bytes(ctx), "hipMalloc(batched matmul partials)");
     if (rc) return rc;
   }
   if (rope_base != 0.0f) {
@@ -1843,5 +1899,5 @@ extern "C" int vtb_hip_reserve(VtbHipCtx* ctx, const VtbHipAttnConfig* cfg, int 
 // and batched-matmul scratch); unchanged by any call that needed no growth.
 extern "C" size_t vtb_hip_scratch_bytes(VtbHipCtx* ctx) {
   if (!ctx) return 0;
-  return ctx->ws_bytes + ctx->n_counters * sizeof(unsigned) + ctx->pf_bytes + ctx->qg_bytes;
+  return ctx->ws_bytes + ctx->n_counters * sizeof(unsigned) + ctx->pf_bytes + ctx->qg_bytes + ctx->qp_bytes;
 }
