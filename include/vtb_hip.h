@@ -301,7 +301,8 @@ void vtb_hip_segment_attn_decode_rope_append(VtbHipSeg *seg, VtbHipBuf *out_buf,
  * rounded to f16, K and V are converted to f16 per 64-key tile with a
  * power-of-two scale where a bf16 tile exceeds f16's range, and P is
  * rounded to f16 for the PV product; the scales are exact and taken back
- * out.  For f32 caches the exact f32 decode kernel runs per query.  The
+ * out.  For f32 caches the products run on the f32 matrix cores (the exact f32
+ * decode kernel once per query for few queries and for head_dim 256).  The
  * context keeps a prefill scratch of about 2*n_kv*head_dim*(pos0+n_tokens)
  * bytes (twice that for bf16), grown on demand. */
 void vtb_hip_segment_attn_prefill(VtbHipSeg *seg, VtbHipBuf *out_buf, VtbHipBuf *q_buf,

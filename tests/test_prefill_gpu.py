@@ -120,6 +120,42 @@ def test_prefill_f32_cache_uses_exact_path(ctx, orc):
     prefill_case(ctx, orc, 8, 2, 64, "f32", 150, pos0=20, window=48, seed=5)
 
 
+@pytest.mark.parametrize("n_heads,n_kv,d,B,pos0,window", [
+    (4, 4, 64, 96, 0, None),      # the fewest queries x KV heads that leave the decode kernel
+    (6, 4, 64, 129, 31, None),    # uneven GQA map, heads not dealt over the XCDs, one query past four tiles
+    (8, 1, 64, 192, 0, None),     # one KV head: chosen by the query count
+    (8, 8, 128, 97, 300, 40),     # a window inside two key tiles
+    (8, 8, 128, 128, 0, 1),       # a window of one row
+    (16, 2, 64, 200, 1000, 64),   # a window of whole tiles, shorter than a wave's stride
+    (7, 1, 128, 385, 5, None),
+])
+def test_prefill_f32_cache_mfma(ctx, orc, n_heads, n_kv, d, B, pos0, window):
+    # the f32 matrix-core kernel, at the f32 bar
+    prefill_case(ctx, orc, n_heads, n_kv, d, "f32", B, pos0=pos0, window=window, seed=B + d, extra_rows=3)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_prefill_f32_cache_values_not_finite(ctx, orc, d):
+    # an inf or NaN value reaches the queries that attend its row, and no
+    # earlier one of its tile
+    import vantablack_amd as vb
+    n_heads = n_kv = 8
+    B = 130
+    q, k, v = (orc.normal(90 + i, B * n_kv * d).reshape(B, n_kv, d) for i in range(3))
+    bad = v.copy()
+    bad[40, 3, 7], bad[100, 0, d - 1] = np.inf, np.nan
+    ob = ctx.alloc(B * n_heads * d * 4)
+    got = []
+    for vals in (v, bad):
+        with ctx.segment() as seg:
+            seg.attn_prefill(ob, ctx.to_device(q), ctx.to_device(k), ctx.to_device(vals), 0, B, 0, vb.NO_WINDOW, n_heads,
+                             n_kv, d, 1.0 / np.sqrt(d), vb.F32)
+        got.append(ctx.download(ob, np.float32, B * n_heads * d).reshape(B, n_heads, d))
+    want = got[0].copy()
+    want[40:, 3, 7], want[100:, 0, d - 1] = np.inf, np.nan
+    assert np.array_equal(got[1], want, equal_nan=True)
+
+
 def test_prefill_row_equals_decode(ctx, orc):
     """prefill.zig:21-23: prefill row b equals a single-token decode at
     position pos0 + b (here: the MFMA prefill vs the f32 decode kernel on

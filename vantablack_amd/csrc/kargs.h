@@ -122,6 +122,21 @@ static_assert(offsetof(PrefillArgs, texp) == 32 && offsetof(PrefillArgs, tstat) 
                   offsetof(PrefillArgs, scale_log2) == 96,
               "PrefillArgs layout");
 
+// Prefill attention over an f32 cache (vtb_prefill_f32_*).
+struct Prefill32Args {
+  const float* q;            // [n_q][n_heads][D]
+  const float* k;            // layer base: row t of KV head h at k + (t * n_kv + h) * D
+  const float* v;
+  float* out;                // [n_q][n_heads][D]
+  int n_q;
+  int n_heads;
+  int n_kv;
+  int pos0;                  // position of query 0; pos0 + n_q < 2^30
+  int window;                // sliding window in rows; <= 0 disables it
+  float scale_log2;          // (1/sqrt(D)) * log2(e)
+};
+static_assert(sizeof(Prefill32Args) == 56 && offsetof(Prefill32Args, n_q) == 32, "Prefill32Args layout");
+
 // Prefill conversion pass (vtb_kvt_*): one workgroup per (64-key tile, KV
 // head), for the tiles [tile_lo, n_tiles) some query attends.  V^T as f16
 // (keys permuted inside each 16-key group) and, for bf16 caches, the keys as

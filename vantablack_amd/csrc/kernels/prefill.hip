@@ -1141,6 +1141,264 @@ __device__ __forceinline__ void prefill_entry(const PrefillArgs& a) {
   }
 }
 
+// ------------------------------------------------------------- f32 caches
+// Causal prefill over an f32 cache on the f32 matrix cores: the flash
+// attention above, with v_mfma_f32_32x32x2_f32 for both products (f32 operands,
+// exact products, f32 sums: no precision to choose).  A workgroup takes 32
+// queries of one head; its four waves take every fourth 32-key tile and are
+// merged through LDS at the end, so that a short prompt's longest row is a
+// quarter as long (512 tokens: four tiles per wave instead of sixteen).
+//   S^T = K Q^T    A = K, B = Q^T.  The instruction sums two k per step, one
+//                  from each lane half; which column of the head that is, is
+//                  free as long as both operands agree: half h takes columns
+//                  [D/2 h, D/2 h + D/2), so a lane's operands are D/2
+//                  consecutive floats of one row, loaded 16 bytes at a time.
+//   O^T += V^T P^T B = P^T: step i takes register i of S^T as it lies, key
+//                  8 (i / 4) + 4 h + i % 4 of the tile from half h, and A =
+//                  V^T reads that key's row, 32 consecutive columns.
+// Operands come straight from the cache (L2 serves the GQA group's heads); the
+// next tile's keys and the next 32 columns of values are loaded under the
+// current products, which take 64 cycles per pair of loads.
+// Measured against the split-K decode kernel once per query, which reads every
+// row from L2 for each query and does its products on the VALU (us per call with
+// the slot writes): 32/4 heads d64, 512 tokens 87 -> 26.5, 32/8 heads d128, 512
+// tokens 152 -> 49 and 2000 tokens 1714 -> 451 (36 TFLOP/s; the matrix cores'
+// f32 rate is 157: a wave's loads, softmax and products take turns, one or two
+// waves per SIMD). Error against 64 bits, relative 2-norm, 512 tokens: 1.25e-7
+// here and 1.19e-7 there at d64, 1.25e-7 and 1.24e-7 at d128; with 1000 or more
+// keys 10-40% less here.
+//
+// Keys masked for some queries of a tile have P = 0, and 0 times a value
+// that is not finite must not reach those queries: in tiles that are masked
+// at all, such values enter the product as 0 and are added by hand, where
+// their key is attended.
+__device__ inline f32x16 mfma_f32(float a, float b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+__device__ inline f32x16 zero16() {
+  f32x16 z;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) z[i] = 0.0f;
+  return z;
+}
+__device__ inline bool is_finite(float x) { return (__builtin_bit_cast(uint32_t, x) & 0x7f800000u) != 0x7f800000u; }
+
+template <int D>
+__device__ __forceinline__ void prefill32_body(const Prefill32Args& a) {
+  constexpr int NT = D / 32, HD = D / 2, LD = D + 4;
+  __shared__ __attribute__((aligned(16))) float s_o[4][32][LD];
+  __shared__ float s_m[4][32], s_l[4][32];
+  const int tid = (int)threadIdx.x, lane = tid & 63, fl = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // An XCD takes consecutive heads (workgroups are dealt over the XCDs in
+  // turn), the longest rows first.
+  const int hx = (int)blockIdx.x;
+  const int head = a.n_heads % 8 == 0 ? (hx & 7) * (a.n_heads >> 3) + (hx >> 3) : hx;
+  const int kvh = (int)((long long)head * a.n_kv / a.n_heads);
+  const int q0 = 32 * (int)(gridDim.y - 1 - blockIdx.y);
+  const int n_rows = a.pos0 + a.n_q;
+  const size_t rs = (size_t)a.n_kv * D;  // floats between rows
+  const float* kb = a.k + (size_t)kvh * D;
+  const float* vb = a.v + (size_t)kvh * D;
+
+  // This lane's query (past the last one: the last one again, not stored).
+  const int qi = q0 + fl < a.n_q ? q0 + fl : a.n_q - 1;
+  const int qp = a.pos0 + qi;
+  auto window_lo = [&](int p) { return a.window > 0 && p >= a.window ? p - a.window + 1 : 0; };
+  const int q_lo = window_lo(qp);
+  const int last = q0 + 31 < a.n_q ? q0 + 31 : a.n_q - 1;
+  const int t_lo = window_lo(a.pos0 + q0) >> 5, t_hi = (a.pos0 + last) >> 5;
+  const int lo_last = window_lo(a.pos0 + last);
+
+  float qf[HD];
+  {
+    const float* qr = a.q + ((size_t)qi * a.n_heads + head) * D + HD * half;
+#pragma unroll
+    for (int j = 0; j < HD / 4; ++j) {
+      const float4 x = *reinterpret_cast<const float4*>(qr + 4 * j);
+      qf[4 * j] = x.x * a.scale_log2;
+      qf[4 * j + 1] = x.y * a.scale_log2;
+      qf[4 * j + 2] = x.z * a.scale_log2;
+      qf[4 * j + 3] = x.w * a.scale_log2;
+    }
+  }
+  // Keys, 32 of a lane's columns at a time: the next 32 (at the end, the next
+  // tile's first) are loaded under a chunk's products; d64's only chunk
+  // after them.
+  constexpr int NCH = HD / 32, KB = NCH > 1 ? 2 : 1;
+  float kf[KB][32];
+  // (a tile's rows through a buffer of its own: rows past n_rows read zeros,
+  // and are masked)
+  auto tile = [&](const float* base, int t) __attribute__((always_inline)) {
+    const int left = n_rows - 32 * t < 32 ? n_rows - 32 * t : 32;
+    return buffer_rsrc(base + (size_t)(32 * t) * rs, (unsigned)left * (unsigned)rs * 4u);
+  };
+  auto f4 = [](__amdgpu_buffer_rsrc_t r, int off) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  };
+  const int koff = 4 * (fl * (int)rs + HD * half), voff = 4 * (4 * half * (int)rs + fl);
+  auto load_k = [&](int t, int c) __attribute__((always_inline)) {
+    const auto r = tile(kb, t);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const f32x4 x = f4(r, koff + 128 * c + 16 * j);
+      kf[c % KB][4 * j] = x.x, kf[c % KB][4 * j + 1] = x.y, kf[c % KB][4 * j + 2] = x.z, kf[c % KB][4 * j + 3] = x.w;
+    }
+  };
+  float vf[2][16];
+  auto load_v = [&](int t, int dt) __attribute__((always_inline)) {
+    const auto r = tile(vb, t);
+    int o = voff;
+    asm volatile("" : "+v"(o));  // (or sixteen row offsets stay in registers across the loop)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      vf[dt & 1][i] = __builtin_bit_cast(
+          float, __builtin_amdgcn_raw_buffer_load_b32(r, o + 4 * (8 * (i >> 2) + (i & 3)) * (int)rs + 128 * dt, 0, 0));
+  };
+
+  f32x16 O[NT];
+#pragma unroll
+  for (int dt = 0; dt < NT; ++dt) O[dt] = zero16();
+  float m = -__builtin_inff(), l = 0.0f;  // l: this lane's keys only
+  if (t_lo + wave <= t_hi) load_k(t_lo + wave, 0);
+  for (int t = t_lo + wave; t <= t_hi; t += 4) {
+    const int t_next = t + 4 <= t_hi ? t + 4 : t;
+    load_v(t, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    // (sums of 8 columns, and of 32, added to each other on the VALU: the
+    // matrix core's running sum over a whole head loses two to four times as
+    // much as the VALU's)
+    f32x16 S;
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      if (NCH > 1) {
+        if (c + 1 < NCH) load_k(t, c + 1); else load_k(t_next, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        f32x16 G;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          f32x16 U = zero16();
+#pragma unroll
+          for (int n = 0; n < 4; ++n) {
+            const int s = 16 * g + 4 * u + n;
+            U = mfma_f32(kf[c % KB][s], qf[32 * c + s], U);
+          }
+#pragma unroll
+          for (int e = 0; e < 16; ++e) G[e] = u == 0 ? U[e] : G[e] + U[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) S[e] = c == 0 && g == 0 ? G[e] : S[e] + G[e];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (NCH == 1) {
+      load_k(t_next, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const bool masked = 32 * t + 31 > a.pos0 + q0 || 32 * t < lo_last;
+    if (masked) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int key = 32 * t + 8 * (i >> 2) + 4 * half + (i & 3);
+        if (key > qp || key < q_lo) S[i] = -__builtin_inff();
+      }
+    }
+    float mx = S[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, S[i]);
+    mx = fmaxf(m, xor_max<32>(mx));
+    const float mu = mx == -__builtin_inff() ? 0.0f : mx;  // (nothing attended yet)
+    const float corr = exp2_fast(m - mu);
+    m = mx;
+    float P[16], sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      P[i] = exp2_fast(S[i] - mu);
+      sum += P[i];
+    }
+    l = l * corr + sum;
+    bool bad = false;
+#pragma unroll
+    for (int dt = 0; dt < NT; ++dt) {
+      if (dt + 1 < NT) load_v(t, dt + 1);
+      if (masked) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (!is_finite(vf[dt & 1][i])) {
+            bad = true;
+            vf[dt & 1][i] = 0.0f;
+          }
+      }
+      f32x16 T;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        f32x16 U = zero16();
+#pragma unroll
+        for (int i = 4 * c; i < 4 * c + 4; ++i) U = mfma_f32(vf[dt & 1][i], P[i], U);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) T[e] = c == 0 ? U[e] : T[e] + U[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) O[dt][e] = fmaf(O[dt][e], corr, T[e]);
+      __builtin_amdgcn_sched_barrier(0);  // (sums of two column tiles at once spill)
+    }
+    if (__any(bad)) {
+      // P by key and query in this wave's own LDS rows, then the values that
+      // are not finite, key by key.
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s_o[wave][8 * (i >> 2) + 4 * half + (i & 3)][fl] = P[i];
+      wait_lds();
+#pragma unroll 1
+      for (int r = 0; r < 32; ++r) {
+        const int key = 32 * t + r;
+        const bool seen = key <= qp && key >= q_lo;
+        const float* vr = vb + (size_t)(key < n_rows ? key : n_rows - 1) * rs;
+        const float pr = s_o[wave][r][fl];
+#pragma unroll
+        for (int dt = 0; dt < NT; ++dt)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const float x = vr[32 * dt + 8 * (e >> 2) + 4 * half + (e & 3)];
+            if (seen && !is_finite(x)) O[dt][e] += pr * x;
+          }
+      }
+      wait_lds();
+    }
+  }
+
+  // Merge: weights 2^(m - M) of the four waves' sums.
+  l = xor_sum<32>(l);
+  if (half == 0) {
+    s_m[wave][fl] = m;
+    s_l[wave][fl] = l;
+  }
+  __syncthreads();
+  const float M = fmaxf(fmaxf(s_m[0][fl], s_m[1][fl]), fmaxf(s_m[2][fl], s_m[3][fl]));
+  // (a wave without tiles has m = -inf, l = 0, O = 0; M is then another's)
+  const float w = m == -__builtin_inff() ? 0.0f : exp2_fast(m - M);
+#pragma unroll
+  for (int dt = 0; dt < NT; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(&s_o[wave][fl][32 * dt + 8 * g + 4 * half]) =
+          f32x4{O[dt][4 * g] * w, O[dt][4 * g + 1] * w, O[dt][4 * g + 2] * w, O[dt][4 * g + 3] * w};
+  if (half == 0) s_l[wave][fl] = l * w;
+  __syncthreads();
+#pragma unroll
+  for (int n = 0; n < D / 32; ++n) {
+    const int idx = tid + 256 * n, qr = idx / (D / 4), c = 4 * (idx % (D / 4));
+    const float L = (s_l[0][qr] + s_l[1][qr]) + (s_l[2][qr] + s_l[3][qr]);
+    f32x4 o = *reinterpret_cast<const f32x4*>(&s_o[0][qr][c]);
+#pragma unroll
+    for (int u = 1; u < 4; ++u) o += *reinterpret_cast<const f32x4*>(&s_o[u][qr][c]);
+    if (q0 + qr < a.n_q)
+      *reinterpret_cast<f32x4*>(a.out + ((size_t)(q0 + qr) * a.n_heads + head) * D + c) = o / L;
+  }
+}
+
 }  // namespace vtb
 
 // The attention kernels are the same for both cache dtypes (f16 operands);
@@ -1174,3 +1432,13 @@ VTB_KVT(bf16, kv_bf16, 256)
 VTB_KVT(f16, kv_f16, 64)
 VTB_KVT(f16, kv_f16, 128)
 VTB_KVT(f16, kv_f16, 256)
+
+// d64 fits two waves per SIMD, d128 one (up to 512 registers).  At d256 the
+// queries and O alone take 256 registers and the rest spills: f32 caches of
+// that width stay with the decode kernel.
+#define VTB_PREFILL_F32(D, W)                                                                      \
+  extern "C" __global__ __launch_bounds__(256, W) void vtb_prefill_f32_d##D(vtb::Prefill32Args a) { \
+    vtb::prefill32_body<D>(a);                                                                     \
+  }
+VTB_PREFILL_F32(64, 2)
+VTB_PREFILL_F32(128, 1)

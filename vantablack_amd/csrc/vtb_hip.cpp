@@ -29,6 +29,7 @@ using vtb::DecodeMergeArgs;
 using vtb::EltArgs;
 using vtb::FillArgs;
 using vtb::GemvArgs;
+using vtb::Prefill32Args;
 using vtb::PrefillArgs;
 using vtb::QGemmArgs;
 using vtb::QReduceArgs;
@@ -90,6 +91,7 @@ struct VtbHipCtx {
   int xcd_map = 0;
   hipFunction_t f_prefill[kNumD] = {};
   hipFunction_t f_prefill_ks[kNumD] = {};  // key-split small-prompt form (d <= 128)
+  hipFunction_t f_prefill_f32[kNumD] = {};
   hipFunction_t f_kvt[kNumKv][kNumD] = {};  // pre-pass per cache dtype (f16, bf16)
   hipFunction_t f_append[kNumKv] = {};
   hipFunction_t f_copy = nullptr;
@@ -642,6 +644,43 @@ int launch_prefill_mfma(VtbHipCtx* ctx, float* out, const float* q, const void* 
                 (unsigned)nt, &a);
 }
 
+// Prefill over an f32 cache: the f32 MFMA kernel, one workgroup per 32 queries
+// of one head; what it does not take (and all that launch_decode refuses) goes
+// to the decode kernel, once per query.
+int launch_prefill_f32(VtbHipCtx* ctx, float* out, const float* q, const void* k, const void* v, size_t n_q,
+                       size_t n_heads, size_t n_kv, size_t head_dim, long long pos0, long long window,
+                       float inv_sqrt_hd) {
+  const int di = d_index(head_dim);
+  // The decode kernel's time grows with the queries times the KV heads (each
+  // query reads every row anew), this one's with the longest row alone until
+  // the CUs are full; a row costs it about 2.5 us per 128 keys at d64. us per
+  // call with the slot writes, here / per query: 32/8 heads d128, 64 tokens 15.9 /
+  // 14.8, 96 16.6 / 19.3, 512 48.7 / 152; 7/1 heads d128, 128 tokens at 2000 112 /
+  // 67, 384 at 2000 125 / 241; 32/4 heads d64, 96 tokens at 2000 62 / 114, 64 at
+  // 500 25.0 / 24.1; 16/16 heads d64, 64 at 500 25 / 19, 128 at 500 26 / 34; 32/32
+  // heads d128, 64 tokens 16.7 / 13.2, 128 18.3 / 22.6.
+  const bool many = n_q >= 3 * head_dim || (n_q >= 96 && n_q * n_kv >= 6 * head_dim);
+  const bool mfma = di >= 0 && ctx->f_prefill_f32[di] && n_heads > 0 && n_kv > 0 && n_kv <= 65535 &&
+                    decode_group_index(n_heads, n_kv) >= 0 && many && n_q <= 65535 && pos0 >= 0 &&
+                    pos0 + (long long)n_q < (1LL << 30) && (long long)(n_kv * head_dim) * 4 * 32 < (1LL << 31) &&
+                    aligned16(k) && aligned16(v) && aligned16(q) && aligned16(out);
+  if (!mfma)
+    return launch_decode(ctx, out, q, k, v, n_q, n_heads, n_kv, head_dim, pos0, window, inv_sqrt_hd, VTB_HIP_F32);
+  Prefill32Args a;
+  memset(&a, 0, sizeof a);
+  a.q = q;
+  a.k = (const float*)k;
+  a.v = (const float*)v;
+  a.out = out;
+  a.n_q = (int)n_q;
+  a.n_heads = (int)n_heads;
+  a.n_kv = (int)n_kv;
+  a.pos0 = (int)pos0;
+  a.window = window > 0 && window < (1LL << 30) ? (int)window : 0;
+  a.scale_log2 = inv_sqrt_hd * 1.4426950408889634f;
+  return launch(ctx, ctx->f_prefill_f32[di], (unsigned)n_heads, (unsigned)((n_q + 31) / 32), 1, 256, &a);
+}
+
 // Quantised GEMV launcher: out[m] = W[m, k] . x.  One workgroup per R rows
 // with one wave per 2048 columns (k <= 32768; R = 4 only up to 16384).  R is
 // 4 where it still gives two workgroups per CU, except for Q6_K with k above
@@ -1024,6 +1063,9 @@ extern "C" VtbHipCtx* vtb_hip_init(void) {
         snprintf(name, sizeof name, "vtb_prefill_d%d", D);
         if (hipModuleGetFunction(&ctx->f_prefill[di], ctx->mod_prefill, name) != hipSuccess)
           ctx->f_prefill[di] = nullptr;
+        snprintf(name, sizeof name, "vtb_prefill_f32_d%d", D);
+        if (D > 128 || hipModuleGetFunction(&ctx->f_prefill_f32[di], ctx->mod_prefill, name) != hipSuccess)
+          ctx->f_prefill_f32[di] = nullptr;
         snprintf(name, sizeof name, "vtb_prefill_ks_d%d", D);
         if (D > 128 || hipModuleGetFunction(&ctx->f_prefill_ks[di], ctx->mod_prefill, name) != hipSuccess)
           ctx->f_prefill_ks[di] = nullptr;
@@ -1453,9 +1495,9 @@ extern "C" void vtb_hip_segment_attn_prefill(VtbHipSeg* seg, VtbHipBuf* out_buf,
   const long long w = window_arg(sliding_window);
   int rc;
   if (dtype == VTB_HIP_F32)
-    rc = launch_decode(ctx, (float*)out_buf->ptr, (const float*)q_buf->ptr,
-                       bptr(k_cache_buf, layer_offset_bytes), bptr(v_cache_buf, layer_offset_bytes),
-                       n_tokens, n_heads, n_kv_heads, head_dim, (long long)pos0, w, inv_sqrt_hd, dtype);
+    rc = launch_prefill_f32(ctx, (float*)out_buf->ptr, (const float*)q_buf->ptr,
+                            bptr(k_cache_buf, layer_offset_bytes), bptr(v_cache_buf, layer_offset_bytes), n_tokens,
+                            n_heads, n_kv_heads, head_dim, (long long)pos0, w, inv_sqrt_hd);
   else
     rc = launch_prefill_mfma(ctx, (float*)out_buf->ptr, (const float*)q_buf->ptr,
                              bptr(k_cache_buf, layer_offset_bytes),
@@ -1807,9 +1849,8 @@ extern "C" int vtb_hip_prefill_attention(VtbHipSeg* seg, VtbHipKvCache* c, const
   const float inv_sqrt_hd = 1.0f / sqrtf((float)cfg->head_dim);
   const long long w = window_arg(cfg->sliding_window);
   if (!rc && c->dtype == VTB_HIP_F32) {
-    rc = launch_decode(ctx, (float*)attn_out->ptr, (const float*)q->ptr, bptr(c->k, lo), bptr(c->v, lo),
-                       n_tokens, cfg->n_heads, cfg->n_kv_heads, cfg->head_dim, (long long)c->pos, w,
-                       inv_sqrt_hd, c->dtype);
+    rc = launch_prefill_f32(ctx, (float*)attn_out->ptr, (const float*)q->ptr, bptr(c->k, lo), bptr(c->v, lo),
+                            n_tokens, cfg->n_heads, cfg->n_kv_heads, cfg->head_dim, (long long)c->pos, w, inv_sqrt_hd);
   } else if (!rc) {
     rc = launch_prefill_mfma(ctx, (float*)attn_out->ptr, (const float*)q->ptr, bptr(c->k, lo), bptr(c->v, lo),
                              n_tokens, cfg->n_heads, cfg->n_kv_heads, cfg->head_dim, (long long)c->pos, w,
