@@ -878,7 +878,6 @@ int launch_qgemm_blocks(VtbHipCtx* ctx, int qk, int nblk, float* const outs[], c
     const size_t n_rb = (ms[b] + kQgRows - 1) / kQgRows;
     if (n_rb * n_tb > 0x3fffffff) return set_err(ctx, VTB_HIP_EUNSUPPORTED, "matmul_batched: too many tokens or rows");
     size_t n_split = std::max((size_t)1, 2 * (size_t)std::max(ctx->cu_count, 1) / (n_rb * n_tb));
-    n_split = (size_t)env_int("VTB_QGEMM_SPLIT", (int)n_split);
     n_split = std::min(n_split, n256);
     const size_t split_blocks = (n256 + n_split - 1) / n_split;
     n_split = (n256 + split_blocks - 1) / split_blocks;
