@@ -405,7 +405,9 @@ int vtb_hip_kv_cache_shrink_to_fit(VtbHipKvCache *cache, size_t new_max_seq);
  * runs the decode kernel, up to max_batch queries) over up to c->max_seq
  * keys or the window; the prefill conversion scratch for a c->max_seq-key
  * context (f16/bf16 caches, max_batch > 0); the batched-matmul activation
- * scratch for max_batch tokens of width max_matmul_k (0: none); the RoPE
+ * scratch for max_batch tokens of width max_matmul_k (0: none); for both of
+ * these the partials of launches split over keys or k (without it such calls
+ * make it, and run unsplit where they cannot: under capture); the RoPE
  * table of rope_base (0: none).  Later calls within these bounds allocate
  * nothing.  Waits for the stream.  5 if a bound is beyond what the kernels
  * take (max_batch > max_seq, max_matmul_k > 32768). */

@@ -456,3 +456,42 @@ def test_prefill_key_split(ctx, orc, monkeypatch, ks, n_heads, n_kv, d, dtype, B
     err = prefill_case(ctx, orc, n_heads, n_kv, d, dtype, B, pos0=pos0, window=window, seed=1200 + B,
                        q_scale=q_scale, v_scale=v_scale, rows=rows, pooled=B * n_heads > 4096)
     print(f"key split={ks} h{n_heads}/{n_kv} d{d} {dtype} B{B} pos0 {pos0} w{window}: rel err {err:.2e}")
+
+
+# Split launches: the key steps of a head's query blocks cut into equal runs,
+# one per workgroup (launch_prefill_mfma picks them where the plain grid leaves
+# most CUs idle), against the unsplit forms (VTB_PREFILL_SPLIT=0) and the
+# oracle: runs within one block and runs over two (d256, 17 blocks at 1995),
+# a partial last block, two to more than eight pieces per block, an odd last
+# tile, a window that starts inside a block, heads that don't fill the merge's
+# workgroups, both two-piece precision forms, and value tiles in units of
+# their own (a ramp, and an all-zero tile).
+@pytest.mark.parametrize("split", ["1", "0"])
+@pytest.mark.parametrize("n_heads,n_kv,d,dtype,B,pos0,window,q_scale,values", [
+    (8, 1, 256, "f16", 2101, 1995, None, 1.0, None),
+    (3, 1, 256, "bf16", 130, 900, None, 1.0, None),
+    (1, 1, 256, "bf16", 33, 1231, None, 1.0, "ramp"),
+    (2, 2, 256, "f16", 200, 1000, 700, 8.0, None),
+    (2, 1, 256, "bf16", 300, 700, None, 1.0, "outliers"),
+    (7, 1, 128, "f16", 65, 2300, None, 1.0, None),
+    (4, 2, 128, "bf16", 200, 1301, None, 1.0, "ramp"),
+    (5, 5, 128, "bf16", 100, 1500, 1111, 8.0, None),
+    (3, 1, 64, "bf16", 1, 2500, None, 1.0, "zero"),
+    (8, 2, 64, "f16", 129, 3000, None, 1.0, "outliers"),
+    (9, 3, 64, "bf16", 300, 2200, 2100, 1.0, None),
+])
+def test_prefill_split_launches(ctx, orc, monkeypatch, split, n_heads, n_kv, d, dtype, B, pos0, window, q_scale,
+                                values):
+    monkeypatch.setenv("VTB_PREFILL_SPLIT", split)
+    v_scale = 1.0
+    if values == "outliers":
+        v_scale = np.ones((1, n_kv, d), np.float32)
+        v_scale[:, :, ::97] = 20.0
+    elif values == "ramp":
+        v_scale = _tile_ramp(pos0 + B, 1.0)
+    elif values == "zero":
+        v_scale = _tile_ramp(pos0 + B, 0.0, zero_tile=3)
+    rows = None if B <= 129 else sorted({0, 1, 63, 64, 127, 128, 129, B // 2, B - 2, B - 1} | set(range(0, B, 97)))
+    err = prefill_case(ctx, orc, n_heads, n_kv, d, dtype, B, pos0=pos0, window=window, seed=1300 + B, q_scale=q_scale,
+                       v_scale=v_scale, rows=rows, pooled=B > 1000)
+    print(f"split={split} h{n_heads}/{n_kv} d{d} {dtype} B{B} pos0 {pos0} w{window}: rel err {err:.2e}")

@@ -106,6 +106,9 @@ struct PrefillArgs {
   float* part_o;             // balance: split-block partials [n_heads][nblk / 2][2][threads][D / 2] f32
   float* part_ml;            // [n_heads][nblk / 2][2][threads][4]: (m, l, E, 0), O in units of 2^E
   unsigned* part_ctr;        // [n_heads][nblk / 2] x 32 arrival counters, zero between launches
+  int part_steps;            // split launches (vtb_prefill_part_*): key steps per run (block_steps)
+  int part_align;            // 1 or part_steps: what a block's steps are filled up to
+  int part_slots;            // partials per head; part_o / part_ml as prefill_write_part lays them
 };
 // PrefillArgs::flags.  kPrefillBalance: paired key ranges (prefill_entry;
 // d256, nblk even).  kPrefillPairOrder: the grid fits two workgroups per
@@ -113,7 +116,7 @@ struct PrefillArgs {
 // blocks complementary to the first half's (prefill_entry).
 constexpr int kPrefillBalance = 1;
 constexpr int kPrefillPairOrder = 2;
-static_assert(sizeof(PrefillArgs) == 128 && offsetof(PrefillArgs, flags) == 100 &&
+static_assert(sizeof(PrefillArgs) == 144 && offsetof(PrefillArgs, flags) == 100 &&
                   offsetof(PrefillArgs, part_o) == 104 && offsetof(PrefillArgs, part_ctr) == 120,
               "PrefillArgs layout");
 static_assert(offsetof(PrefillArgs, texp) == 32 && offsetof(PrefillArgs, tstat) == 40 &&

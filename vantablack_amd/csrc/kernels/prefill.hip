@@ -490,6 +490,48 @@ __device__ __forceinline__ void item_keys(const PrefillArgs& a, int qb, long lon
   if (a.window > 0 && q_lo >= a.window && q_lo - a.window + 1 > kbeg) kbeg = q_lo - a.window + 1;
 }
 
+// Split launches (PART): the key steps of a head's query blocks, the last
+// block's first, are one line that the head's workgroups cut into equal runs
+// of a.part_steps: a run holds the end of one block, whole blocks and the
+// start of another, or, where every block is filled up to a multiple of
+// part_align = part_steps, a piece of one block.  A step is a key tile, or the
+// two tiles the key-split form takes at a time.  block_steps: the steps
+// [0, n) of block qb, from key tile t0 on (those past its keys are not run).
+struct BlockSteps {
+  int t0, n;
+};
+template <int D, int BM>
+__device__ __forceinline__ BlockSteps block_steps(const PrefillArgs& a, int qb) {
+  constexpr int BN = prefill_block_n(D), ST = BM == 64 ? 2 : 1;
+  const int q0 = (int)a.pos0 + qb * BM, m1 = (qb + 1) * BM < a.n_q ? (qb + 1) * BM : a.n_q;
+  const int kend = (int)a.pos0 + m1;
+  const int kbeg = a.window > 0 && q0 >= a.window ? q0 - (int)a.window + 1 : 0;
+  const int t0 = kbeg / BN;
+  const int n = ((kend + BN - 1) / BN - t0 + ST - 1) / ST;
+  return BlockSteps{t0, (int)((unsigned)(n + a.part_align - 1) / (unsigned)a.part_align) * a.part_align};
+}
+
+// A piece's unnormalised partial for vtb_prefill_merge_*: O in units of 2^E
+// as rows [slot][BM][D], (m, l, E) as [slot][BM][4]; slot = head * part_slots +
+// run + blocks before this one (no two pieces of a head share it), r the
+// query's row in its block.
+template <int D, int BM>
+__device__ __forceinline__ void prefill_write_part(const PrefillArgs& a, int h, int qb, int slot, int r, int hi,
+                                                   const f32x16 (&o)[D / 32], float m_ref, float l_run, int E) {
+  float l0, l1;
+  lane_halves(l_run, l0, l1);
+  if (qb * BM + r >= a.n_q) return;
+  const long long row = ((long long)h * a.part_slots + slot) * BM + r;
+  float* op = a.part_o + row * D + 4 * hi;
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<f32x4*>(op + 32 * dt + 8 * g) =
+          f32x4{o[dt][4 * g], o[dt][4 * g + 1], o[dt][4 * g + 2], o[dt][4 * g + 3]};
+  if (hi == 0) *reinterpret_cast<f32x4*>(a.part_ml + row * 4) = f32x4{m_ref, l0 + l1, (float)E, 0.0f};
+}
+
 // A KV head's f16 key rows and V^T rows, as the tile DMA reads them.
 struct TileSrc {
   const char* kbase;
@@ -510,7 +552,7 @@ __device__ __forceinline__ TileSrc tile_src(const PrefillArgs& a, int kvh) {
 // The entry has issued the DMA of the item's first key tile into stage 0
 // (key-split: its first two tiles, into k0/v0 and k2/v2) and the load of
 // that tile's exponents (x_first; key-split: the wave's own tile's).
-template <int D, int NW, bool XQ, bool XP, bool KSPLIT>
+template <int D, int NW, bool XQ, bool XP, bool KSPLIT, bool PART>
 __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const int h, const int qb, const int kvh,
                                              const f16x8 (&qf)[D / 16], const f16x8 (&ql)[D / 16],
                                              const int eq, PrefillLds<D>& lds, const long long k_lo,
@@ -913,7 +955,12 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const int h, 
     E = Em;
   }
 
-  if constexpr (kBalanced<D>) {
+  if constexpr (PART) {
+    if (piece >= 0) {
+      prefill_write_part<D, BM>(a, h, qb, piece, wsb * 32 + lc, hi, o, m_ref, l_run, E);
+      return;
+    }
+  } else if constexpr (kBalanced<D>) {
     if (piece >= 0 && !prefill_merge_pieces<D, NW>(a, h, qb, piece, o, m_ref, l_run, E)) return;
   }
 
@@ -932,7 +979,7 @@ __device__ __forceinline__ void prefill_body(const PrefillArgs& a, const int h, 
 //       |v - out|, so outlier values carry it into the output.
 // Keys of bf16 caches are exact in f16 (per-tile power-of-two scale), f16
 // keys are the cache itself; P's rounding enters the output through V only.
-template <int D, int NW, bool KSPLIT = false>
+template <int D, int NW, bool KSPLIT = false, bool PART = false>
 __device__ __forceinline__ void prefill_entry(const PrefillArgs& a) {
   constexpr int KS = D / 16;
   constexpr int BM = prefill_item_queries(NW, KSPLIT);
@@ -952,13 +999,13 @@ __device__ __forceinline__ void prefill_entry(const PrefillArgs& a) {
                     (lchar*)s_k2, (lchar*)s_k3, (lchar*)s_v2, (lchar*)s_v3};
   const int nblk = gridDim.y;
   int h, w;
+  int rank;  // position of the workgroup's query block in dispatch order
   {
     // Workgroups are dispatched round-robin over the 8 XCDs in linear order.
     // When the heads split evenly, XCD x gets heads [x*hpx, (x+1)*hpx) --
     // with GQA these share KV heads, so each XCD's L2 holds fewer K/V tiles
     // -- and every XCD takes its longest (last) query blocks first.
     const int i = blockIdx.y * gridDim.x + blockIdx.x;
-    int rank;  // position of the workgroup's query block in dispatch order
     if (a.n_heads % 8 == 0) {
       const int hpx = a.n_heads / 8, j = i / 8;
       h = (i % 8) * hpx + j % hpx;
@@ -988,7 +1035,19 @@ __device__ __forceinline__ void prefill_entry(const PrefillArgs& a) {
   };
   int n_items = 1, qb0 = w, qb1 = 0, pc0 = -1;
   long long lo0 = 0, hi0 = 1LL << 62;
-  if (kBalanced<D> && (a.flags & kPrefillBalance)) {
+  // Split launches: run `rank` of the head's line starts at step p_lo of
+  // block qb0, p_left steps of it are left (block_steps).
+  BlockSteps pb{};
+  int p_lo = 0, p_left = 0;
+  if constexpr (PART) {
+    pb = block_steps<D, BM>(a, qb0 = (a.n_q - 1) / BM);
+    p_lo = rank * a.part_steps;
+    p_left = a.part_steps;
+    while (p_lo >= pb.n) {
+      p_lo -= pb.n;
+      pb = block_steps<D, BM>(a, --qb0);
+    }
+  } else if (kBalanced<D> && (a.flags & kPrefillBalance)) {
     const int p = w >> 1, c = nblk - 1 - p, b = p;
     const long long kc = kend_of(c), kb = kend_of(b);
     const long long S = (kb + kc) / 2 / BN * BN;
@@ -1006,9 +1065,21 @@ __device__ __forceinline__ void prefill_entry(const PrefillArgs& a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hi = lane >> 5, lc = lane & 31;
   for (int it = 0; it < n_items; ++it) {
-    const int qb = it == 0 ? qb0 : qb1;
-    const int piece = it == 0 ? pc0 : -1;
-    const long long k_lo = it == 0 ? lo0 : 0, k_hi = it == 0 ? hi0 : (1LL << 62);
+    int qb = it == 0 ? qb0 : qb1;
+    int piece = it == 0 ? pc0 : -1;
+    long long k_lo = it == 0 ? lo0 : 0, k_hi = it == 0 ? hi0 : (1LL << 62);
+    if constexpr (PART) {
+      qb = qb0;
+      const int n = pb.n - p_lo < p_left ? pb.n - p_lo : p_left;
+      constexpr int SK = (KSPLIT ? 2 : 1) * BN;  // keys per step
+      piece = n == pb.n ? -1 : rank + (a.n_q - 1) / BM - qb;
+      k_lo = (long long)pb.t0 * BN + (long long)p_lo * SK;
+      k_hi = k_lo + (long long)n * SK;
+      p_left -= n;
+      p_lo = 0;
+      n_items = p_left > 0 && qb0 > 0 ? it + 2 : it + 1;
+      if (qb0 > 0) pb = block_steps<D, BM>(a, --qb0);
+    }
     if (it > 0) __syncthreads();  // the previous item's LDS reads are done
     // The item's keys; the DMA of its first key tile into stage 0 goes out
     // before the q and statistics loads, so the three latencies overlap
@@ -1133,11 +1204,11 @@ __device__ __forceinline__ void prefill_entry(const PrefillArgs& a) {
     // kernel made the register allocator spill VGPRs in the d128 and d256
     // kernels.
     if (xp)
-      prefill_body<D, NW, true, true, KSPLIT>(a, h, qb, kvh, qf, ql, eq, lds, k_lo, k_hi, piece, x_first);
+      prefill_body<D, NW, true, true, KSPLIT, PART>(a, h, qb, kvh, qf, ql, eq, lds, k_lo, k_hi, piece, x_first);
     else if (xq)
-      prefill_body<D, NW, true, false, KSPLIT>(a, h, qb, kvh, qf, ql, eq, lds, k_lo, k_hi, piece, x_first);
+      prefill_body<D, NW, true, false, KSPLIT, PART>(a, h, qb, kvh, qf, ql, eq, lds, k_lo, k_hi, piece, x_first);
     else
-      prefill_body<D, NW, false, false, KSPLIT>(a, h, qb, kvh, qf, ql, eq, lds, k_lo, k_hi, piece, x_first);
+      prefill_body<D, NW, false, false, KSPLIT, PART>(a, h, qb, kvh, qf, ql, eq, lds, k_lo, k_hi, piece, x_first);
   }
 }
 
@@ -1399,6 +1470,70 @@ __device__ __forceinline__ void prefill32_body(const Prefill32Args& a) {
   }
 }
 
+// The pieces of every split query block (PART launches) put together: grid y
+// the query, D / 4 lanes per head, four dims each; the pieces are added in
+// key order, each scaled from its own reference max and value unit to the
+// row's largest.  A piece whose keys the query may not attend holds l = 0.
+template <int N>
+struct PieceBatch {
+  static constexpr int n = N;
+};
+template <int D, int BM>
+__device__ __forceinline__ void prefill_merge_body(const PrefillArgs& a) {
+  constexpr int HPW = 1024 / D;  // heads per workgroup of 256
+  const int mq = blockIdx.y, h = blockIdx.x * HPW + threadIdx.x / (D / 4), c = threadIdx.x % (D / 4) * 4;
+  if (h >= a.n_heads) return;
+  const int qb = mq / BM, last = (a.n_q - 1) / BM;
+  int off = 0;
+  for (int q = last; q > qb; --q) off += block_steps<D, BM>(a, q).n;
+  const int run = off / a.part_steps;  // the first run in the block
+  const int pieces = (off + block_steps<D, BM>(a, qb).n - 1) / a.part_steps - run + 1;
+  if (pieces == 1) return;  // the run wrote the whole block
+  const long long row = ((long long)h * a.part_slots + run + last - qb) * BM + (mq - qb * BM);
+  const f32x4* ml = reinterpret_cast<const f32x4*>(a.part_ml) + row;
+  const float* op = a.part_o + row * D + c;
+  float M = -INFINITY, E = -INFINITY, l = 0.0f;
+  f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+  // U pieces' loads in flight; past the last piece it is read again and not
+  // counted.
+  auto add = [&](auto batch, int i0) {
+    constexpr int U = decltype(batch)::n;
+    f32x4 x[U], v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long long i = i0 + u < pieces ? i0 + u : pieces - 1;
+      x[u] = ml[i * BM];
+      v[u] = *reinterpret_cast<const f32x4*>(op + i * BM * D);
+    }
+    float Mn = M, En = E;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      Mn = fmaxf(Mn, x[u][0]);
+      if (x[u][0] != -INFINITY) En = fmaxf(En, x[u][2]);
+    }
+    const float f0 = M == -INFINITY ? 0.0f : exp2_fast(M - Mn);
+    const float g0 = M == -INFINITY ? 0.0f : f0 * pow2_diff((int)(E - En));
+    l *= f0;
+    o *= g0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool live = i0 + u < pieces && x[u][0] != -INFINITY;
+      const float f = live ? exp2_fast(x[u][0] - Mn) : 0.0f;
+      const float g = live ? f * pow2_diff((int)(x[u][2] - En)) : 0.0f;
+      l += x[u][1] * f;
+      o += v[u] * g;
+    }
+    M = Mn;
+    E = En;
+  };
+  if (pieces <= 3)
+    add(PieceBatch<3>{}, 0);
+  else
+    for (int i0 = 0; i0 < pieces; i0 += 8) add(PieceBatch<8>{}, i0);
+  const float inv = (1.0f / l) * pow2_diff((int)E);
+  *reinterpret_cast<f32x4*>(a.out + ((long long)mq * a.n_heads + h) * D + c) = o * inv;
+}
+
 }  // namespace vtb
 
 // The attention kernels are the same for both cache dtypes (f16 operands);
@@ -1426,6 +1561,27 @@ VTB_PREFILL(128)
 VTB_PREFILL(256)
 VTB_PREFILL_KS(64)
 VTB_PREFILL_KS(128)
+// Split launches (plan_prefill_split): d256 in the plain form, d <= 128
+// key-split; then the kernel that puts the pieces together.  The plain grid of
+// a chunk has a workgroup per 64 or 128 queries and head, each over every key
+// before it: most CUs idle, and the matrix cores wait on one workgroup's
+// chain.  us per call with the slot writes and the pre-pass, unsplit / split:
+// d256 8/1 heads f16, 2101 queries at 1995 (136 workgroups) 169 / 117, 512 at
+// 8000 325 / 76, 64 at 4000 158 / 37, 100 at 16000 585 / 58; d128 32/8 heads
+// bf16, 64 at 4000 83 / 42, 100 at 16000 255 / 101.  The first: 104 in the
+// attention (0.5 PFLOP/s of the causal products; the key tiles' LDS reads and
+// the softmax between the products bound it), 15 in the merge (50 MB of
+// partials).
+#define VTB_PREFILL_PART(D, KS)                                                                      \
+  extern "C" __global__ __launch_bounds__(256, 1) void vtb_prefill_part_d##D(vtb::PrefillArgs a) {   \
+    vtb::prefill_entry<D, 4, KS, true>(a);                                                           \
+  }                                                                                                  \
+  extern "C" __global__ __launch_bounds__(256) void vtb_prefill_merge_d##D(vtb::PrefillArgs a) {     \
+    vtb::prefill_merge_body<D, vtb::prefill_item_queries(4, KS)>(a);                                 \
+  }
+VTB_PREFILL_PART(64, true)
+VTB_PREFILL_PART(128, true)
+VTB_PREFILL_PART(256, false)
 VTB_KVT(bf16, kv_bf16, 64)
 VTB_KVT(bf16, kv_bf16, 128)
 VTB_KVT(bf16, kv_bf16, 256)

@@ -91,6 +91,8 @@ struct VtbHipCtx {
   int xcd_map = 0;
   hipFunction_t f_prefill[kNumD] = {};
   hipFunction_t f_prefill_ks[kNumD] = {};  // key-split small-prompt form (d <= 128)
+  hipFunction_t f_prefill_part[kNumD] = {};   // split launches
+  hipFunction_t f_prefill_merge[kNumD] = {};  // and their pieces put together
   hipFunction_t f_prefill_f32[kNumD] = {};
   hipFunction_t f_kvt[kNumKv][kNumD] = {};  // pre-pass per cache dtype (f16, bf16)
   hipFunction_t f_append[kNumKv] = {};
@@ -118,9 +120,8 @@ struct VtbHipCtx {
   // Batched-matmul activation scratch, written by vtb_xsplit (qgemm_scratch).
   void* qg = nullptr;
   size_t qg_bytes = 0;
-  // Partials of matmuls split along k (qgemm_part_bytes).
+  // Partials of split launches (partials_ready).
   void* qp = nullptr;
-  size_t qp_bytes = 0;
   // RoPE inverse-frequency tables 1/base^(2j/d) on the device, one per
   // (base, head_dim) seen; the host copy stays alive for the async upload.
   struct RopeTable {
@@ -524,6 +525,83 @@ int ensure_scratch(VtbHipCtx* ctx, void** buf, size_t* have, size_t need, const 
   return VTB_HIP_OK;
 }
 
+// The partials of launches that split a reduction over more workgroups: one
+// buffer per context, written and consumed by the kernels of one call, of one
+// size for good (recorded graphs hold its address).  The largest: 128 queries at
+// head_dim 256, two per CU; a matmul's are 64 KiB each, two per CU.
+size_t partials_bytes(const VtbHipCtx* ctx) {
+  return 2 * (size_t)std::max(ctx->cu_count, 1) * 128 * (256 + 4) * sizeof(float);
+}
+// False where it is not there and cannot be made -- under capture, or out of
+// memory -- and the caller then launches unsplit.
+bool partials_ready(VtbHipCtx* ctx) {
+  if (ctx->qp) return true;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone &&
+      hipMalloc(&ctx->qp, partials_bytes(ctx)) == hipSuccess)
+    return true;
+  ctx->qp = nullptr;
+  (void)hipGetLastError();
+  return false;
+}
+
+// Split prefill launches (vtb_prefill_part_*, block_steps): the key steps of a
+// head's query blocks in runs of `steps`, one per workgroup, as many as the
+// CUs take at once; 0: not split.
+struct PrefillSplit {
+  int steps = 0, align = 1, runs = 0, slots = 0;
+  size_t ml = 0;  // partials: O rows, then (m, l, E) rows at byte ml
+};
+PrefillSplit plan_prefill_split(const VtbHipCtx* ctx, size_t n_q, size_t n_heads, size_t head_dim, size_t bm,
+                                long long pos0, long long window, bool balance) {
+  PrefillSplit r;
+  const long long bn = vtb::prefill_block_n((int)head_dim), st = bm == 64 ? 2 : 1;
+  const long long nblk = (long long)((n_q + bm - 1) / bm);
+  const long long want = std::max(ctx->cu_count, 1) / (long long)n_heads;
+  if (nblk > want) return r;
+  // As block_steps counts them.
+  auto steps_of = [&](long long b) {
+    const long long q_lo = pos0 + b * (long long)bm, kend = pos0 + std::min((b + 1) * (long long)bm, (long long)n_q);
+    const long long kbeg = window > 0 && q_lo >= window ? q_lo - window + 1 : 0;
+    return ((kend + bn - 1) / bn - kbeg / bn + st - 1) / st;
+  };
+  auto total = [&](long long align) {
+    long long n = 0;
+    for (long long b = 0; b < nblk; ++b) n += (steps_of(b) + align - 1) / align;
+    return n;
+  };
+  long long longest = 0;
+  for (long long b = 0; b < nblk; ++b) longest = std::max(longest, steps_of(b));
+  // Runs within one block: the fewest steps whose runs fit.
+  const long long even = (total(1) + want - 1) / want;
+  long long aligned = even, hi = longest;
+  while (aligned < hi) {
+    const long long t = (aligned + hi) / 2;
+    if (total(t) <= want) hi = t; else aligned = t + 1;
+  }
+  // A run over two blocks loads queries, statistics and the first tile anew
+  // and leaves two partials, so it has to save some steps.  8/1 heads d256: 512
+  // tokens at 8000 (33 steps / 34 aligned) 87 / 80 us, 256 at 1000 (3 / 3) 49 /
+  // 42, 2101 at 1995 (51 / 71) 117 / 133.
+  const bool over = aligned - even > 6;
+  const long long steps = over ? even : aligned;
+  // The second launch and the partials cost what about ten steps do.  Unsplit /
+  // split: d256 8/1 heads 33 tokens at 300 (11 steps / 1) 31.3 / 25.0 us, 128 at 100
+  // (8 / 1) 32.2 / 31.2, 16/8 heads bf16 34.3 / 38.8; d128 7/1 heads 256 at 1000 (10 /
+  // 2) 35.6 / 28.8, 32/8 heads (10 / 5) 39.3 / 41.4; d64 32/4 heads 256 at 1000 (10 / 5)
+  // 26.1 / 27.5, 64 at 4000 (32 / 4) 50.7 / 25.7.
+  // Runs over two blocks need twice that: d128 7/1 heads 2101 at 1995 (32 / 22)
+  // 82 / 89.
+  const long long unsplit = balance ? (longest + steps_of(0)) / 2 : longest;
+  if (unsplit - steps < (over ? 2 : 1) * (head_dim <= 64 ? 12 : head_dim <= 128 ? 8 : 10)) return r;
+  r.steps = (int)steps;
+  r.align = over ? 1 : r.steps;
+  r.runs = (int)(over ? (total(1) + steps - 1) / steps : total(steps));
+  r.slots = r.runs + (int)nblk - 1;
+  r.ml = n_heads * (size_t)r.slots * bm * head_dim * sizeof(float);
+  return r;
+}
+
 // MFMA prefill: q is f32 (prefill.zig's s.q); k/v the layer base of an f16
 // or bf16 cache.  One pre-pass (V^T, tile statistics and, for bf16, the
 // scaled f16 keys and tile exponents) over the 64-key tiles from the window
@@ -559,8 +637,16 @@ int launch_prefill_mfma(VtbHipCtx* ctx, float* out, const float* q, const void* 
   // an even block count and causal ranges not cut by a window.  C5 (4096
   // tokens, 8/1 heads): 140 against 214 us per call.  VTB_PREFILL_BALANCE=0
   // turns it off.
-  const bool balance = !ks && env_flag("VTB_PREFILL_BALANCE", true) && head_dim >= 256 && nblk >= 2 &&
-                       nblk % 2 == 0 && (window <= 0 || window >= pos0 + (long long)n_q);
+  bool balance = !ks && env_flag("VTB_PREFILL_BALANCE", true) && head_dim >= 256 && nblk >= 2 &&
+                 nblk % 2 == 0 && (window <= 0 || window >= pos0 + (long long)n_q);
+  // Chunks of a prompt far from its start, whose few blocks have long key
+  // ranges: VTB_PREFILL_SPLIT=0 turns it off.
+  PrefillSplit split;
+  if ((ks || head_dim >= 256) && ctx->f_prefill_part[di] && env_flag("VTB_PREFILL_SPLIT", true)) {
+    split = plan_prefill_split(ctx, n_q, n_heads, head_dim, bm, pos0, window, balance);
+    if (split.steps && !partials_ready(ctx)) split = PrefillSplit();
+    if (split.steps) balance = false;
+  }
   const size_t nt = 256;
   // Pre-pass over keys [0, pos0 + n_q), padded to whole 64-key tiles, from
   // the tile of the first query's window start on (no query reads earlier
@@ -637,6 +723,18 @@ int launch_prefill_mfma(VtbHipCtx* ctx, float* out, const float* q, const void* 
     a.part_o = (float*)(base + ps.bal_o);
     a.part_ml = (float*)(base + ps.bal_ml);
     a.part_ctr = ctx->counters;
+  }
+  if (split.steps) {
+    a.part_steps = split.steps;
+    a.part_align = split.align;
+    a.part_slots = split.slots;
+    a.part_o = (float*)ctx->qp;
+    a.part_ml = (float*)((char*)ctx->qp + split.ml);
+    rc = launch(ctx, ctx->f_prefill_part[di], (unsigned)n_heads, (unsigned)split.runs, 1, (unsigned)nt, &a);
+    if (rc) return rc;
+    const size_t heads_per_wg = 1024 / head_dim;
+    return launch(ctx, ctx->f_prefill_merge[di], (unsigned)((n_heads + heads_per_wg - 1) / heads_per_wg), (unsigned)n_q,
+                  1, 256, &a);
   }
   // x = head (fastest), y = query block: the longest (causal) blocks of every
   // head are dispatched first.
@@ -820,9 +918,8 @@ QgemmScratch qgemm_scratch(size_t B, size_t k) {
   return q;
 }
 constexpr size_t kQgRows = 256;  // rows of a workgroup
-// Partials of the matmuls whose k range is split: one tile of f32 per
-// workgroup, at most two workgroups per CU.
-size_t qgemm_part_bytes(VtbHipCtx* ctx) { return 2 * (size_t)std::max(ctx->cu_count, 1) * 64 * kQgRows * sizeof(float); }
+// Matmuls split along k leave one 64 KiB tile of f32 per workgroup in the
+// context's partials, at most two workgroups per CU.
 
 // Batched quantised matmul launcher: out[B][m] = acts[B][k] . W^T.  The
 // pre-pass scales each token by a power of two and splits it into two f16
@@ -879,11 +976,11 @@ int launch_qgemm_blocks(VtbHipCtx* ctx, int qk, int nblk, float* const outs[], c
     if (n_rb * n_tb > 0x3fffffff) return set_err(ctx, VTB_HIP_EUNSUPPORTED, "matmul_batched: too many tokens or rows");
     size_t n_split = std::max((size_t)1, 2 * (size_t)std::max(ctx->cu_count, 1) / (n_rb * n_tb));
     n_split = std::min(n_split, n256);
-    const size_t split_blocks = (n256 + n_split - 1) / n_split;
+    size_t split_blocks = (n256 + n_split - 1) / n_split;
     n_split = (n256 + split_blocks - 1) / split_blocks;
-    if (n_split > 1) {
-      rc = ensure_scratch(ctx, &ctx->qp, &ctx->qp_bytes, qgemm_part_bytes(ctx), "hipMalloc(batched matmul partials)");
-      if (rc) return rc;
+    if (n_split > 1 && !partials_ready(ctx)) {
+      n_split = 1;
+      split_blocks = n256;
     }
     QGemmArgs a;
     memset(&a, 0, sizeof a);
@@ -1062,6 +1159,12 @@ extern "C" VtbHipCtx* vtb_hip_init(void) {
         snprintf(name, sizeof name, "vtb_prefill_d%d", D);
         if (hipModuleGetFunction(&ctx->f_prefill[di], ctx->mod_prefill, name) != hipSuccess)
           ctx->f_prefill[di] = nullptr;
+        snprintf(name, sizeof name, "vtb_prefill_part_d%d", D);
+        if (hipModuleGetFunction(&ctx->f_prefill_part[di], ctx->mod_prefill, name) != hipSuccess)
+          ctx->f_prefill_part[di] = nullptr;
+        snprintf(name, sizeof name, "vtb_prefill_merge_d%d", D);
+        if (hipModuleGetFunction(&ctx->f_prefill_merge[di], ctx->mod_prefill, name) != hipSuccess)
+          ctx->f_prefill_part[di] = nullptr;
         snprintf(name, sizeof name, "vtb_prefill_f32_d%d", D);
         if (D > 128 || hipModuleGetFunction(&ctx->f_prefill_f32[di], ctx->mod_prefill, name) != hipSuccess)
           ctx->f_prefill_f32[di] = nullptr;
@@ -1901,6 +2004,7 @@ extern "C" int vtb_hip_reserve(VtbHipCtx* ctx, const VtbHipAttnConfig* cfg, int 
   int rc = ensure_workspace(ctx, ws, ctr);
   if (rc) return rc;
   if (kv_dtype != VTB_HIP_F32 && max_batch > 0) {
+    partials_ready(ctx);
     const long long vt_ld = ((long long)max_seq + 63) / 64 * 64;
     // With balanced pairs enabled, the d256 kernel's partials for up to
     // max_batch queries.
@@ -1923,8 +2027,7 @@ extern "C" int vtb_hip_reserve(VtbHipCtx* ctx, const VtbHipAttnConfig* cfg, int 
     rc = ensure_scratch(ctx, &ctx->qg, &ctx->qg_bytes, qgemm_scratch(max_batch, max_matmul_k).bytes,
                         "hipMalloc(batched matmul scratch)");
     if (rc) return rc;
-    rc = ensure_scratch(ctx, &ctx->qp, &ctx->qp_bytes, qgemm_part_bytes(ctx), "hipMalloc(batched matmul partials)");
-    if (rc) return rc;
+    partials_ready(ctx);
   }
   if (rope_base != 0.0f) {
     RopeArgs ra;
@@ -1939,5 +2042,6 @@ extern "C" int vtb_hip_reserve(VtbHipCtx* ctx, const VtbHipAttnConfig* cfg, int 
 // and batched-matmul scratch); unchanged by any call that needed no growth.
 extern "C" size_t vtb_hip_scratch_bytes(VtbHipCtx* ctx) {
   if (!ctx) return 0;
-  return ctx->ws_bytes + ctx->n_counters * sizeof(unsigned) + ctx->pf_bytes + ctx->qg_bytes + ctx->qp_bytes;
+  return ctx->ws_bytes + ctx->n_counters * sizeof(unsigned) + ctx->pf_bytes + ctx->qg_bytes +
+         (ctx->qp ? partials_bytes(ctx) : 0);
 }
