@@ -396,6 +396,29 @@ VtbHipBuf *vtb_hip_kv_cache_v(VtbHipKvCache *cache);
  * unlike the Metal path).  0, or 4 if new_max_seq < pos. */
 int vtb_hip_kv_cache_shrink_to_fit(VtbHipKvCache *cache, size_t new_max_seq);
 
+/* ---- a token through a whole model: gpuLayerStep per layer (forward.zig:419-513)
+ * and gpuFinalStep (:515-520), one call.  x holds the token's embedding and is
+ * left as the normalised residual stream, logits[vocab_size] the projection,
+ * row pos of every layer's K/V slab ([n_layers][max_seq][n_kv_heads][head_dim]
+ * of kv_dtype) the token's.  Norms and residual adds run inside the GEMVs next
+ * to them; xb, xb2, q, k_cur, v_cur, attn_out, gate, up and ffn_out are scratch
+ * of the layer's sizes whose contents afterwards are unspecified.  Offsets are
+ * bytes into weights; kinds 0 q8_0, 1 q4_k, 2 q5_k, 3 q6_k; activation 0 silu,
+ * 1 gelu_approx. */
+typedef struct VtbHipTokenLayer {
+  size_t attn_norm, wq, wk, wv, wo, ffn_norm, wgate, wup, wdown;
+  size_t kind_q, kind_k, kind_v, kind_o, kind_gate, kind_up, kind_down;
+} VtbHipTokenLayer;
+typedef struct VtbHipTokenStep {
+  VtbHipBuf *x, *xb, *xb2, *q, *k_cur, *v_cur, *attn_out, *gate, *up, *ffn_out, *logits, *weights, *kv_k, *kv_v;
+  size_t dim, n_heads, n_kv_heads, head_dim, ffn_dim, max_seq, sliding_window, pos;
+  const VtbHipTokenLayer *layers;
+  size_t n_layers, output_norm, output, output_kind, vocab_size;
+  int kv_dtype, rope_half, activation;
+  float rope_base, rms_eps;
+} VtbHipTokenStep;
+void vtb_hip_segment_token_step(VtbHipSeg *seg, const VtbHipTokenStep *step);
+
 /* ---- scratch reservation: the counterpart of prefill.zig Scratch.init
  * (prefill.zig:67-88), which sizes the batch scratch for B tokens and the
  * score rows for max_seq once, before the first forward.  Grows, once, every

@@ -228,6 +228,91 @@ def test_model_decode_matches_cpu_layer_steps(ctx, orc, variant, path):
             b.release()
 
 
+class _Launches:
+    """A segment without token_step: gpu_token_step encodes its launches one
+    by one."""
+
+    def __init__(self, seg):
+        self._seg = seg
+
+    def __getattr__(self, name):
+        return getattr(self._seg, name)
+
+
+# The native token step (norms inside the projections that read x, residual
+# adds inside those that produce it, formats mixed in one launch) against the
+# single launches, over an f32 cache.  Widths: below one 2048-column slice
+# (four row waves per workgroup), exactly one with the rows for R = 4 and 2,
+# and two waves along k of which the second is partly past k; every format,
+# gate and up of one format and of two, both activations.  Both sides are f32
+# and differ by the order of a few roundings of 2^-24 per activation (the
+# norm's scale before or after the dot), averaged over k: 1e-5 of the largest
+# value leaves a factor of 20 for two layers.
+@pytest.mark.parametrize("dim,heads,n_kv,d,ffn,act,kinds", [
+    (256, 4, 2, 64, 512, "silu", ("q4_k", "q5_k", "q6_k", "q8_0", "q4_k", "q8_0", "q5_k")),
+    (512, 2, 1, 256, 2304, "gelu_approx", ("q8_0", "q8_0", "q4_k", "q6_k", "q6_k", "q6_k", "q8_0")),
+    (2048, 32, 4, 64, 5632, "silu", ("q4_k", "q4_k", "q6_k", "q4_k", "q4_k", "q4_k", "q6_k")),
+    (2304, 18, 6, 128, 1280, "gelu_approx", ("q5_k", "q6_k", "q6_k", "q5_k", "q5_k", "q5_k", "q4_k")),
+    (2304, 18, 3, 128, 768, "silu", ("q6_k", "q4_k", "q8_0", "q6_k", "q5_k", "q6_k", "q6_k")),
+])
+def test_token_step_matches_its_launches(ctx, dim, heads, n_kv, d, ffn, act, kinds):
+    import vantablack_amd as vb
+    from vantablack_amd.layer import LayerConfig, LayerOffsets, LayerScratch, gpu_token_step
+    c = LayerConfig(dim=dim, n_heads=heads, n_kv_heads=n_kv, head_dim=d, ffn_dim=ffn, max_seq=8, activation=act,
+                    sliding_window=2, kv_dtype=vb.F32)
+    rng = np.random.default_rng(dim + ffn)
+    vocab, kv_dim, n_layers = 515, n_kv * d, 2
+    parts, pos = [], 0
+
+    def put(a):
+        nonlocal pos
+        b = np.ascontiguousarray(a).view(np.uint8).reshape(-1)
+        parts.append(np.concatenate([b, np.zeros(-b.size % 32, np.uint8)]))
+        pos += parts[-1].size
+        return pos - parts[-1].size
+
+    def norm():
+        return put((1 + 0.1 * rng.standard_normal(dim)).astype(np.float32))
+
+    shapes = [(dim, dim), (kv_dim, dim), (kv_dim, dim), (dim, dim), (ffn, dim), (ffn, dim), (dim, ffn)]
+    offs = []
+    for l in range(n_layers):
+        w = [put(random_weights(kd, m, k, seed=31 * l + i)) for i, (kd, (m, k)) in enumerate(zip(kinds, shapes))]
+        offs.append(LayerOffsets(norm(), *w[:4], norm(), *w[4:], *kinds))
+    out_norm, out = norm(), put(random_weights("q6_k", vocab, dim, seed=5))
+    wbuf = ctx.to_device(np.concatenate(parts))
+    xs = rng.standard_normal((4, dim)).astype(np.float32)
+    res = []
+    for native in (True, False):
+        s = LayerScratch(ctx, c, vocab)
+        kv = [ctx.to_device(np.zeros(n_layers * c.max_seq * kv_dim, np.float32)) for _ in range(2)]
+        got = []
+        for p in range(4):
+            ctx.upload(s.x, xs[p])
+            with ctx.segment() as seg:
+                gpu_token_step(seg if native else _Launches(seg), s, wbuf, offs, *kv, c, p, out_norm, out, "q6_k", vocab)
+            ctx.wait_idle()
+            got.append((ctx.download(s.x, np.float32, dim), ctx.download(s.logits, np.float32, vocab)))
+        got.append([ctx.download(b, np.float32, n_layers * c.max_seq * kv_dim) for b in kv])
+        res.append(got)
+        s.release()
+        for b in kv:
+            b.release()
+    for a, b in zip(*res):
+        for u, v in zip(a, b):
+            err = np.max(np.abs(u - v)) / np.max(np.abs(v))
+            print(f"dim {dim} ffn {ffn}: {err:.1e}")
+            assert err <= 1e-5
+    # what the launches refuse, the native step refuses
+    with pytest.raises(vb.HipError):
+        s = LayerScratch(ctx, c, vocab)
+        with ctx.segment() as seg:
+            gpu_token_step(seg, s, wbuf, [LayerOffsets(pos, *(0,) * 8, *kinds)], wbuf, wbuf, c, 0, out_norm, out, "q6_k",
+                           vocab)
+    s.release()
+    wbuf.release()
+
+
 @pytest.mark.parametrize("kv", ["f16", "bf16"])
 @pytest.mark.parametrize("variant", ["llama_q4_k", "mistral_q8_0_gqa_window"])
 def test_model_decode_half_cache(ctx, orc, variant, kv):

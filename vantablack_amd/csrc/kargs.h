@@ -218,9 +218,13 @@ struct GemvArgs {
   // workgroup takes rows [R/2 wg, +R/2) of both W_gate (w) and W_up (w1) and
   // writes act(gate) * up to out; 1 = silu (swiglu), 2 = gelu_approx.
   int gated;
+  float eps;            // vtb_gemvn_*: activations x * norm_w / sqrt(mean x^2 + eps)
+  const float* norm_w;  // [k], 4-byte aligned
+  const float* add;     // out = add + W x (may be out); null: none
+  int kind, kind1, kind2;  // vtb_gemvn_*: the blocks' formats
   int pad;
 };
-static_assert(sizeof(GemvArgs) == 112, "GemvArgs layout");
+static_assert(sizeof(GemvArgs) == 144, "GemvArgs layout");
 static_assert(offsetof(GemvArgs, w1) == 56 && offsetof(GemvArgs, w2) == 80 && offsetof(GemvArgs, gated) == 104,
               "GemvArgs layout");
 

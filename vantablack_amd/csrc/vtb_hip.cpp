@@ -98,7 +98,8 @@ struct VtbHipCtx {
   hipFunction_t f_append[kNumKv] = {};
   hipFunction_t f_copy = nullptr;
   hipFunction_t f_fill = nullptr;
-  hipFunction_t f_gemv[kNumQuant][kNumGemvR] = {};  // vtb_gemv_<kind>_r<1|2|4>
+  hipFunction_t f_gemv[kNumQuant][kNumGemvR] = {};   // vtb_gemv_<kind>_r<1|2|4>
+  hipFunction_t f_gemvn[2][kNumGemvR] = {};  // vtb_gemvn_r*, vtb_gemvn_s_r*: of the rmsnorm of x
   hipFunction_t f_xsplit = nullptr, f_xsplit_1 = nullptr, f_qgemm_reduce = nullptr;
   hipModule_t mod_layer = nullptr;  // rmsnorm, swiglu, gelu_approx, residual_add
   hipFunction_t f_rmsnorm = nullptr, f_swiglu = nullptr, f_gelu = nullptr, f_resadd = nullptr, f_addnorm = nullptr;
@@ -787,7 +788,7 @@ int launch_prefill_f32(VtbHipCtx* ctx, float* out, const float* q, const void* k
 // Up to three row blocks of one format sharing x go in one launch
 // (launch_gemv_blocks); R is chosen on the total rows.
 int launch_gemv_blocks(VtbHipCtx* ctx, int qk, int nblk, float* const outs[], const void* const ws[],
-                       const size_t ms[], const float* x, size_t k) {
+                       const size_t ms[], const float* x, size_t k, const float* add = nullptr) {
   if (qk < 0 || qk >= kNumQuant) return set_err(ctx, VTB_HIP_EINVAL, "bad quant kind");
   if (nblk < 1 || nblk > 3) return set_err(ctx, VTB_HIP_EINVAL, "matmul: 1 to 3 row blocks");
   if (k == 0 || k % kQuantBlockElems[qk] != 0)
@@ -831,6 +832,7 @@ int launch_gemv_blocks(VtbHipCtx* ctx, int qk, int nblk, float* const outs[], co
   a.k = (int)k;
   a.row_bytes = (int)row_bytes;
   a.nblk = nblk;
+  a.add = add;
   size_t grid = (ms[0] + R - 1) / R;
   if (nblk > 1) {
     a.wg1 = (int)grid;
@@ -895,11 +897,69 @@ int launch_gemv_gated(VtbHipCtx* ctx, int qk, int act, float* out, const void* w
   return launch(ctx, ctx->f_gemv[qk][ri], (unsigned)((m + RH - 1) / RH), 1, 1, 64 * waves, &a, lds);
 }
 
-int launch_gemv(VtbHipCtx* ctx, int qk, float* out, const void* w, const float* x, size_t m, size_t k) {
+int launch_gemv(VtbHipCtx* ctx, int qk, float* out, const void* w, const float* x, size_t m, size_t k,
+                const float* add = nullptr) {
   float* const outs[1] = {out};
   const void* const ws[1] = {w};
   const size_t ms[1] = {m};
-  return launch_gemv_blocks(ctx, qk, 1, outs, ws, ms, x, k);
+  return launch_gemv_blocks(ctx, qk, 1, outs, ws, ms, x, k, add);
+}
+
+// One to three projections (gated: the pair gate, up into one output) of the
+// rmsnorm of x, each in its own format: the norm, and the projections that no
+// single vtb_gemv launch takes, without launches of their own.  The caller has
+// checked shapes, ranges and alignment (token_step).
+struct GemvBlock {
+  int qk;
+  float* out;
+  const void* w;
+  size_t m;
+};
+int launch_gemv_norm(VtbHipCtx* ctx, const GemvBlock* b, int nblk, int gated, const float* x, size_t k,
+                     const float* norm_w, float eps) {
+  // One wave per 2048 columns, R rows per workgroup; k <= 2048 puts four row
+  // waves in a workgroup instead, which share the norm's and the activations'
+  // loads.  R as for the plain GEMV: the largest that leaves two waves per
+  // SIMD's worth of workgroups on the CUs.
+  const bool few = k <= 2048;
+  const size_t rw = few ? 4 : 1, cus = (size_t)std::max(ctx->cu_count, 1);
+  auto groups = [&](size_t m, size_t R) { return (m + rw * R - 1) / (rw * R); };
+  int ri = 0;
+  for (int i = kNumGemvR - 1; i >= 0; --i) {
+    const size_t R = (size_t)kGemvRs[i];
+    if (R == 4 && k > 8 * 2048) continue;
+    if (gated && R == 1) break;
+    ri = i;
+    size_t n = gated ? groups(b[0].m, R / 2) : 0;
+    for (int j = 0; j < nblk && !gated; ++j) n += groups(b[j].m, R);
+    if (n >= (few ? 1 : 2) * cus) break;
+  }
+  const size_t R = (size_t)kGemvRs[ri];
+  GemvArgs a;
+  memset(&a, 0, sizeof a);
+  auto wbytes = [&](const GemvBlock& g) {
+    return (unsigned)((g.m * (k / kQuantBlockElems[g.qk] * kQuantBlockBytes[g.qk]) + 3) & ~(size_t)3);
+  };
+  a.x = x;
+  a.k = (int)k;
+  a.norm_w = norm_w;
+  a.eps = eps;
+  a.nblk = gated ? 1 : nblk;
+  a.gated = gated;
+  a.w = (const uint8_t*)b[0].w, a.out = b[0].out, a.w_bytes = wbytes(b[0]), a.m = (int)b[0].m, a.kind = b[0].qk;
+  size_t grid = groups(b[0].m, gated ? R / 2 : R);
+  if (nblk > 1) {
+    a.w1 = (const uint8_t*)b[1].w, a.out1 = b[1].out, a.w_bytes1 = wbytes(b[1]), a.m1 = (int)b[1].m, a.kind1 = b[1].qk;
+    a.wg1 = (int)grid;
+    if (!gated) grid += groups(b[1].m, R);
+  }
+  if (nblk > 2) {
+    a.w2 = (const uint8_t*)b[2].w, a.out2 = b[2].out, a.w_bytes2 = wbytes(b[2]), a.m2 = (int)b[2].m, a.kind2 = b[2].qk;
+    a.wg2 = (int)grid;
+    grid += groups(b[2].m, R);
+  }
+  const unsigned kwaves = (unsigned)((k + 2047) / 2048);
+  return launch(ctx, ctx->f_gemvn[few][ri], (unsigned)grid, 1, 1, 64 * (few ? 4 : kwaves), &a, kwaves * 8u * (64u + 4u) * 16u);
 }
 
 // Batched-matmul scratch for B tokens of width k, in whole tiles: tokens Bp (B
@@ -1185,6 +1245,10 @@ extern "C" VtbHipCtx* vtb_hip_init(void) {
     for (int ri = 0; ok && ri < kNumGemvR; ++ri) {
       snprintf(name, sizeof name, "vtb_gemv_%s_r%d", kQuantNames[qk], kGemvRs[ri]);
       ok = hipModuleGetFunction(&ctx->f_gemv[qk][ri], ctx->mod_gemv, name) == hipSuccess;
+      for (int few = 0; ok && few < 2; ++few) {
+        snprintf(name, sizeof name, "vtb_gemvn_%sr%d", few ? "s_" : "", kGemvRs[ri]);
+        ok = hipModuleGetFunction(&ctx->f_gemvn[few][ri], ctx->mod_gemv, name) == hipSuccess;
+      }
     }
   ok = ok && hipModuleGetFunction(&ctx->f_xsplit, ctx->mod_qgemm, "vtb_xsplit") == hipSuccess;
   ok = ok && hipModuleGetFunction(&ctx->f_xsplit_1, ctx->mod_qgemm, "vtb_xsplit_1") == hipSuccess;
@@ -1611,14 +1675,14 @@ extern "C" void vtb_hip_segment_attn_prefill(VtbHipSeg* seg, VtbHipBuf* out_buf,
 // ============================================================== quantised GEMV
 
 static int matmul_entry(VtbHipCtx* ctx, int qk, VtbHipBuf* out_buf, VtbHipBuf* w_buf, size_t w_offset,
-                        VtbHipBuf* acts_buf, size_t m, size_t k) {
+                        VtbHipBuf* acts_buf, size_t m, size_t k, const float* add = nullptr) {
   if (!ctx || !out_buf || !w_buf || !acts_buf) return VTB_HIP_EINVAL;
   if (m == 0 || k == 0 || k % kQuantBlockElems[qk] != 0 || m > ((size_t)1 << 31) || k > ((size_t)1 << 31))
     return set_err(ctx, VTB_HIP_EINVAL, "matmul: bad shape");
   const size_t row_bytes = k / kQuantBlockElems[qk] * kQuantBlockBytes[qk];
   if (!buf_ok(w_buf, w_offset, m * row_bytes) || !buf_ok(acts_buf, 0, k * 4) || !buf_ok(out_buf, 0, m * 4))
     return set_err(ctx, VTB_HIP_EINVAL, "matmul: buffer too small");
-  return launch_gemv(ctx, qk, (float*)out_buf->ptr, bptr(w_buf, w_offset), (const float*)acts_buf->ptr, m, k);
+  return launch_gemv(ctx, qk, (float*)out_buf->ptr, bptr(w_buf, w_offset), (const float*)acts_buf->ptr, m, k, add);
 }
 
 #define VTB_MATMUL_ENTRIES(NAME, QK)                                                                     \
@@ -1675,22 +1739,25 @@ static int matmul3_entry(VtbHipCtx* ctx, int qk, VtbHipBuf* out0, size_t w_off0,
                                 acts_buf, k));                                                            \
   }
 
+static int matmul_gated_entry(VtbHipCtx* ctx, int qk, VtbHipBuf* out_buf, VtbHipBuf* w_buf, size_t w_off_gate,
+                              size_t w_off_up, VtbHipBuf* acts_buf, size_t m, size_t k, int activation) {
+  if (!out_buf || !w_buf || !acts_buf || m == 0 || k == 0 || k % kQuantBlockElems[qk] != 0 || m > ((size_t)1 << 31) ||
+      k > ((size_t)1 << 31))
+    return set_err(ctx, VTB_HIP_EINVAL, "matmul_gated: bad shape");
+  const size_t rb = k / kQuantBlockElems[qk] * kQuantBlockBytes[qk];
+  if (!buf_ok(w_buf, w_off_gate, m * rb) || !buf_ok(w_buf, w_off_up, m * rb) || !buf_ok(acts_buf, 0, k * 4) ||
+      !buf_ok(out_buf, 0, m * 4))
+    return set_err(ctx, VTB_HIP_EINVAL, "matmul_gated: buffer too small");
+  return launch_gemv_gated(ctx, qk, activation == 0 ? 1 : (activation == 1 ? 2 : 0), (float*)out_buf->ptr,
+                           bptr(w_buf, w_off_gate), bptr(w_buf, w_off_up), (const float*)acts_buf->ptr, m, k);
+}
+
 #define VTB_MATMUL_GATED_ENTRY(NAME, QK)                                                                  \
   extern "C" void vtb_hip_segment_matmul_gated_##NAME(VtbHipSeg* seg, VtbHipBuf* out_buf, VtbHipBuf* w_buf,    \
                                                       size_t w_off_gate, size_t w_off_up, VtbHipBuf* acts_buf, \
                                                       size_t m, size_t k, int activation) {                    \
     if (!seg) return;                                                                                      \
-    VtbHipCtx* ctx = seg->ctx;                                                                             \
-    if (!out_buf || !w_buf || !acts_buf || m == 0 || k == 0 || k % kQuantBlockElems[QK] != 0 ||            \
-        m > ((size_t)1 << 31) || k > ((size_t)1 << 31))                                                    \
-      return seg_note(seg, set_err(ctx, VTB_HIP_EINVAL, "matmul_gated: bad shape"));                       \
-    const size_t rb = k / kQuantBlockElems[QK] * kQuantBlockBytes[QK];                                     \
-    if (!buf_ok(w_buf, w_off_gate, m * rb) || !buf_ok(w_buf, w_off_up, m * rb) || !buf_ok(acts_buf, 0, k * 4) || \
-        !buf_ok(out_buf, 0, m * 4))                                                                        \
-      return seg_note(seg, set_err(ctx, VTB_HIP_EINVAL, "matmul_gated: buffer too small"));                \
-    seg_note(seg, launch_gemv_gated(ctx, QK, activation == 0 ? 1 : (activation == 1 ? 2 : 0),             \
-                                    (float*)out_buf->ptr, bptr(w_buf, w_off_gate), bptr(w_buf, w_off_up),  \
-                                    (const float*)acts_buf->ptr, m, k));                                   \
+    seg_note(seg, matmul_gated_entry(seg->ctx, QK, out_buf, w_buf, w_off_gate, w_off_up, acts_buf, m, k, activation)); \
   }
 
 VTB_MATMUL_GATED_ENTRY(q8_0, 0)
@@ -1774,6 +1841,88 @@ VTB_MATMUL_BATCHED_ENTRIES(q8_0, 0)
 VTB_MATMUL_BATCHED_ENTRIES(q4_k, 1)
 VTB_MATMUL_BATCHED_ENTRIES(q5_k, 2)
 VTB_MATMUL_BATCHED_ENTRIES(q6_k, 3)
+
+// One token through every layer and the logits (gpuLayerStep per layer, then
+// gpuFinalStep), each rmsnorm inside the projections that read it and each
+// residual add inside the projection that produces it: five launches per
+// layer, whatever the formats.
+extern "C" void vtb_hip_segment_token_step(VtbHipSeg* seg, const VtbHipTokenStep* t) {
+  if (!seg) return;
+  VtbHipCtx* ctx = seg->ctx;
+  if (!t || (t->n_layers && !t->layers)) return seg_note(seg, set_err(ctx, VTB_HIP_EINVAL, "token_step: no layers"));
+  const size_t kv_dim = t->n_kv_heads * t->head_dim, row_bytes = kv_dim * (size_t)kv_bytes(t->kv_dtype);
+  const size_t wstart = t->sliding_window == VTB_HIP_NO_WINDOW || t->pos < t->sliding_window
+                            ? 0 : t->pos - t->sliding_window + 1;
+  const float inv_sqrt_hd = (float)(1.0 / std::sqrt((double)t->head_dim));
+  const bool gelu = t->activation == 1;
+  struct Proj {
+    size_t kind;
+    VtbHipBuf* out;
+    size_t off, m;
+  };
+  auto matmul = [&](const Proj& p, VtbHipBuf* acts, size_t k, const float* add = nullptr) {
+    seg_note(seg, p.kind < (size_t)kNumQuant
+                      ? matmul_entry(ctx, (int)p.kind, p.out, t->weights, p.off, acts, p.m, k, add)
+                      : set_err(ctx, VTB_HIP_EINVAL, "token_step: bad quant kind"));
+  };
+  // Projections of the normalised x (gated: the pair into p[0].out); false,
+  // with nothing launched, for a shape, range or alignment that the single
+  // launches refuse or take another way.
+  auto norm_matmul = [&](size_t norm, const Proj* p, int n, int act) -> bool {
+    const size_t k = t->dim;
+    if (k == 0 || k > 16 * 2048 || norm % 4 || !buf_ok(t->x, 0, k * 4) || !buf_ok(t->xb, 0, k * 4) ||
+        !buf_ok(t->weights, norm, k * 4) || !aligned16(t->x->ptr) || (uintptr_t)bptr(t->weights, norm) % 4)
+      return false;
+    GemvBlock b[3];
+    for (int i = 0; i < n; ++i) {
+      if (p[i].kind >= (size_t)kNumQuant || k % kQuantBlockElems[p[i].kind] != 0) return false;
+      const size_t rb = k / kQuantBlockElems[p[i].kind] * kQuantBlockBytes[p[i].kind], m = p[i].m;
+      if (m == 0 || m > 0x7fff0000 / rb || !buf_ok(t->weights, p[i].off, m * rb) ||
+          (!(act && i) && !buf_ok(p[i].out, 0, m * 4)))
+        return false;
+      b[i] = GemvBlock{(int)p[i].kind, act && i ? nullptr : (float*)p[i].out->ptr, bptr(t->weights, p[i].off), m};
+      if ((uintptr_t)b[i].w % 4 != 0) return false;
+    }
+    seg_note(seg, launch_gemv_norm(ctx, b, n, act, (const float*)t->x->ptr, k, (const float*)bptr(t->weights, norm),
+                                   t->rms_eps));
+    return true;
+  };
+  // x += W acts (tmp: where the reference's separate add reads W acts from).
+  auto matmul_add = [&](size_t kind, VtbHipBuf* tmp, size_t off, VtbHipBuf* acts, size_t k) {
+    if (!buf_ok(t->x, 0, t->dim * 4) || !buf_ok(tmp, 0, t->dim * 4))
+      return seg_note(seg, set_err(ctx, VTB_HIP_EINVAL, "token_step: buffer too small"));
+    matmul(Proj{kind, t->x, off, t->dim}, acts, k, (const float*)t->x->ptr);
+  };
+  for (size_t l = 0; l < t->n_layers; ++l) {
+    const VtbHipTokenLayer& L = t->layers[l];
+    const Proj qkv[3] = {{L.kind_q, t->q, L.wq, t->dim}, {L.kind_k, t->k_cur, L.wk, kv_dim},
+                         {L.kind_v, t->v_cur, L.wv, kv_dim}};
+    if (!norm_matmul(L.attn_norm, qkv, 3, 0)) {
+      vtb_hip_segment_rmsnorm(seg, t->xb, t->x, t->weights, L.attn_norm, t->dim, t->rms_eps);
+      for (const Proj& p : qkv) matmul(p, t->xb, t->dim);
+    }
+    const size_t off = l * t->max_seq * row_bytes + wstart * row_bytes;
+    vtb_hip_segment_attn_decode_rope_append(seg, t->attn_out, t->q, t->kv_k, off, t->kv_v, off, t->k_cur, t->v_cur,
+                                            t->n_heads, t->n_kv_heads, t->head_dim, t->pos + 1 - wstart, inv_sqrt_hd,
+                                            t->kv_dtype, t->pos, t->rope_base, t->rope_half);
+    matmul_add(L.kind_o, t->xb2, L.wo, t->attn_out, t->dim);
+    const bool gated = L.kind_gate == L.kind_up;  // gate takes the pair's output
+    const Proj ffn[2] = {{L.kind_gate, t->gate, L.wgate, t->ffn_dim}, {L.kind_up, t->up, L.wup, t->ffn_dim}};
+    if (!gated || !norm_matmul(L.ffn_norm, ffn, 2, gelu ? 2 : 1)) {
+      if (gated || !norm_matmul(L.ffn_norm, ffn, 2, 0)) {
+        vtb_hip_segment_rmsnorm(seg, t->xb, t->x, t->weights, L.ffn_norm, t->dim, t->rms_eps);
+        for (const Proj& p : ffn) matmul(p, t->xb, t->dim);
+      }
+      if (gelu)
+        vtb_hip_segment_gelu_approx(seg, t->gate, t->up, t->ffn_dim);
+      else
+        vtb_hip_segment_swiglu(seg, t->gate, t->up, t->ffn_dim);
+    }
+    matmul_add(L.kind_down, t->ffn_out, L.wdown, t->gate, t->ffn_dim);
+  }
+  vtb_hip_segment_rmsnorm(seg, t->x, t->x, t->weights, t->output_norm, t->dim, t->rms_eps);
+  matmul(Proj{t->output_kind, t->logits, t->output, t->vocab_size}, t->x, t->dim);
+}
 
 // ============================================================== KvCache
 

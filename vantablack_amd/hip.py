@@ -65,6 +65,20 @@ class AttnConfigC(ctypes.Structure):
 
 # Every symbol include/vtb_hip.h declares, with its ctypes signature.
 _P, _S, _I, _F = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_float
+
+
+class TokenStepC(ctypes.Structure):
+    """VtbHipTokenStep."""
+    _fields_ = ([(n, _P) for n in ("x", "xb", "xb2", "q", "k_cur", "v_cur", "attn_out", "gate", "up", "ffn_out",
+                                   "logits", "weights", "kv_k", "kv_v")]
+                + [(n, _S) for n in ("dim", "n_heads", "n_kv_heads", "head_dim", "ffn_dim", "max_seq",
+                                     "sliding_window", "pos")]
+                + [("layers", _P)]
+                + [(n, _S) for n in ("n_layers", "output_norm", "output", "output_kind", "vocab_size")]
+                + [(n, _I) for n in ("kv_dtype", "rope_half", "activation")]
+                + [("rope_base", _F), ("rms_eps", _F)])
+
+
 SIGNATURES = {
     "vtb_hip_init": ([], _P),
     "vtb_hip_destroy": ([_P], None),
@@ -99,6 +113,7 @@ SIGNATURES = {
     "vtb_hip_segment_matmul_batched3_q4_k": ([_P, _P, _S, _S, _P, _S, _S, _P, _S, _S, _P, _P, _S, _S], None),
     "vtb_hip_segment_matmul_batched3_q5_k": ([_P, _P, _S, _S, _P, _S, _S, _P, _S, _S, _P, _P, _S, _S], None),
     "vtb_hip_segment_matmul_batched3_q6_k": ([_P, _P, _S, _S, _P, _S, _S, _P, _S, _S, _P, _P, _S, _S], None),
+    "vtb_hip_segment_token_step": ([_P, _P], None),
     "vtb_hip_segment_matmul3_q8_0": ([_P, _P, _S, _S, _P, _S, _S, _P, _S, _S, _P, _P, _S], None),
     "vtb_hip_segment_matmul3_q4_k": ([_P, _P, _S, _S, _P, _S, _S, _P, _S, _S, _P, _P, _S], None),
     "vtb_hip_segment_matmul3_q5_k": ([_P, _P, _S, _S, _P, _S, _S, _P, _S, _S, _P, _P, _S], None),
@@ -173,6 +188,7 @@ def _check(ctx_h, rc: int, what: str):
 
 
 QUANT_KINDS = ("q8_0", "q4_k", "q5_k", "q6_k")
+_QUANT_INDEX = {kind: i for i, kind in enumerate(QUANT_KINDS)}
 
 
 @dataclasses.dataclass
@@ -297,6 +313,31 @@ class Segment:
                                                       v_cur.h, n_heads, n_kv_heads, head_dim, seq_len,
                                                       inv_sqrt_hd, kv_dtype, rope_pos, rope_base,
                                                       1 if rope_half else 0)
+
+    def token_step(self, s, weights: Buffer, offs, kv_k: Buffer, kv_v: Buffer, c, pos: int, output_norm_off: int,
+                   output_off: int, output_kind: str, vocab_size: int):
+        """layer.gpu_token_step in one call, the norms and residual adds inside
+        the GEMVs next to them (vtb_hip_segment_token_step)."""
+        for o in offs:
+            for kind in (o.kind_q, o.kind_k, o.kind_v, o.kind_o, o.kind_gate, o.kind_up, o.kind_down):
+                if kind not in _QUANT_INDEX:
+                    raise ValueError(f"unknown quant kind {kind!r}")
+        if output_kind not in _QUANT_INDEX:
+            raise ValueError(f"unknown quant kind {output_kind!r}")
+        DTYPE_BYTES[c.kv_dtype]  # KeyError for an unknown cache dtype
+        ix = _QUANT_INDEX
+        flat = []
+        for o in offs:
+            flat += (o.attn_norm, o.wq, o.wk, o.wv, o.wo, o.ffn_norm, o.wgate, o.wup, o.wdown, ix[o.kind_q],
+                     ix[o.kind_k], ix[o.kind_v], ix[o.kind_o], ix[o.kind_gate], ix[o.kind_up], ix[o.kind_down])
+        layers = (_S * len(flat))(*flat)
+        step = TokenStepC(s.x.h, s.xb.h, s.xb2.h, s.q.h, s.k_cur.h, s.v_cur.h, s.attn_out.h, s.gate.h, s.up.h,
+                          s.ffn_out.h, s.logits.h, weights.h, kv_k.h, kv_v.h, c.dim, c.n_heads, c.n_kv_heads,
+                          c.head_dim, c.ffn_dim, c.max_seq, c.sliding_window, pos, ctypes.cast(layers, _P), len(offs),
+                          output_norm_off, output_off, ix[output_kind], vocab_size, c.kv_dtype,
+                          1 if c.rope_half else 0, {"silu": 0, "gelu_approx": 1}[c.activation], c.rope_base,
+                          c.rms_eps)
+        lib().vtb_hip_segment_token_step(self.h, ctypes.byref(step))
 
     def matmul_quant(self, kind: str, out: Buffer, w: Buffer, w_offset: int, acts: Buffer, m: int, k: int):
         """out = W @ acts for m rows of `kind` blocks (q8_0, q4_k, q5_k, q6_k):

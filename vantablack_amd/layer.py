@@ -18,7 +18,9 @@ each residual add fused into the rmsnorm that follows it
 launch (vtb_hip_segment_matmul3_<kind>) and the gate/up GEMVs with the
 activation in one launch (vtb_hip_segment_matmul_gated_<kind>) when the
 projections share a format: 7 launches per layer instead of 13, the same
-arithmetic per output.
+arithmetic per output.  A hip.Segment encodes it in one native call of 5
+launches per layer (vtb_hip_segment_token_step): each norm inside the
+projections that read it, each residual add inside the one that produces it.
 
 The sliding window is the reference's caller-side offset shift
 (forward.zig:470-480): the K/V base moves to the window's first row and the
@@ -159,8 +161,15 @@ def gpu_token_step(seg, s: LayerScratch, weights, offs, kv_k, kv_v, c: LayerConf
     """Every layer in offs, then gpuFinalStep, for the token at pos (s.x holds
     its embedding); leaves the normalised x in s.x and the logits in s.logits.
     Each residual add runs fused with the rmsnorm after it, and Q/K/V and
-    gate/up (+ activation) run grouped when their formats match."""
+    gate/up (+ activation) run grouped when their formats match.  A hip.Segment
+    encodes it in one native call, where the norms and adds run inside the
+    GEMVs next to them (Segment.token_step); any other segment gets the launches
+    below one by one."""
     _check(c, pos)
+    native = getattr(type(seg), "token_step", None)
+    if native:
+        native(seg, s, weights, offs, kv_k, kv_v, c, pos, output_norm_off, output_off, output_kind, vocab_size)
+        return
     for layer, off in enumerate(offs):
         if layer == 0:
             seg.rmsnorm(s.xb, s.x, weights, off.attn_norm, c.dim, c.rms_eps)
