@@ -55,10 +55,10 @@
 //
 // Measured (before: 128 x 128 tiles, weights unpacked into LDS, sub-blocks
 // scaled on the VALU; us per call with its pre-pass): Q4_K 14336 x 4096, 2048
-// tokens 794 -> 524 (459 TFLOP/s of the reference's flops, 0.95 PFLOP/s of
+// tokens 794 -> 506 (475 TFLOP/s of the reference's flops, 0.98 PFLOP/s of
 // MFMA work, where a plain f16 matrix product of the library runs at
 // 1.1-1.2); Q5_K 797 -> 537, Q8_0 736 -> 585, Q6_K 903 -> 720; 4096 x 4096 with 33
-// tokens, Q8_0: 122 -> 24.  With the unpacking, the flush into acc or the
+// tokens, Q8_0: 122 -> 21.  With the unpacking, the flush into acc or the
 // staging of x taken out (timing only) Q4_K takes 471, 465 and 456 us against
 // 501: no one part bounds it.
 #include "common.h"
@@ -99,6 +99,7 @@ __device__ __forceinline__ void xsplit_body(const XSplitArgs& a) {
     float mx = 0.0f;
     if (t0 + tl < a.B) {
       const float* row = a.x + (size_t)(t0 + tl) * a.k;
+#pragma unroll 4
       for (int c = 4 * (NT >= 4 ? lane : tid); c < a.k; c += 256 * WPT) {
         const float4 v = *reinterpret_cast<const float4*>(row + c);
         mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
@@ -271,7 +272,7 @@ template <bool FIVE> struct QfK45 {
   // sc (q - centre).  A quant in the top mantissa bits of an f16 whose ulp
   // there is 1 is bias + q: Q4_K bits 4..7 under 0x5400 (64 + q), Q5_K bits
   // 3..7 under 0x5800 (128 + q).
-  __device__ static f16x8 unpack(const Raw& raw, const Head& hd, const Sc& sc, int j, int i) {
+  __device__ static f16x8 unpack(const Raw& raw, const Head& hd, const Sc& sc, int j, int i, uint32_t m, uint32_t bias) {
     const int hi = i >> 1;
     uint32_t p[4];
 #pragma unroll
@@ -284,8 +285,8 @@ template <bool FIVE> struct QfK45 {
         p[2 * d] = qperm(0x58585858u, u, 0x04020400u);
         p[2 * d + 1] = qperm(0x58585858u, u, 0x04030401u);
       } else {
-        p[2 * d] = ((hi ? v : v << 4) & 0x00F000F0u) | 0x54005400u;
-        p[2 * d + 1] = ((hi ? v >> 8 : v >> 4) & 0x00F000F0u) | 0x54005400u;
+        p[2 * d] = ((hi ? v : v << 4) & m) | bias;
+        p[2 * d + 1] = ((hi ? v >> 8 : v >> 4) & m) | bias;
       }
     }
     return frag(as_u(pk_fma(as_h2(p[0]), sc.a, sc.b)), as_u(pk_fma(as_h2(p[1]), sc.a, sc.b)),
@@ -526,6 +527,13 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& a) {
     return *reinterpret_cast<const f16x8*>(&s_x[0][0] + slot * XB + 8192 * tt + 4096 * p + 1024 * i + 16 * lane);
   };
 
+  // Q4_K's mask and bias, one in an SGPR and one in a VGPR and out of the
+  // compiler's sight: as literals they make two instructions of every and-or
+  // (14336 x 4096, 2048 tokens: 514 us, 506 so).
+  uint32_t k_mask = 0x00F000F0u, k_bias = 0x54005400u;
+  asm("" : "+s"(k_mask));
+  asm("" : "+v"(k_bias));
+
   load_x(c_lo);
   load_head(b_lo);
   load_w(c_lo);
@@ -597,7 +605,7 @@ __device__ __forceinline__ void qgemm_body(const QGemmArgs& a) {
           if constexpr (KIND == QG6_K)
             F::unpack(raw[rt], F::scales(hd[rt], j, i >> 1, half), j, i, w[rt], wl[rt]);
           else
-            w[rt] = F::unpack(raw[rt], hd[rt], F::scales(hd[rt], j, i >> 1), j, i);
+            w[rt] = F::unpack(raw[rt], hd[rt], F::scales(hd[rt], j, i >> 1), j, i, k_mask, k_bias);
         }
 #pragma unroll
         for (int p = 0; p < 2; ++p)
@@ -693,8 +701,8 @@ extern "C" __global__ __launch_bounds__(256) void vtb_xsplit(vtb::XSplitArgs a) 
 extern "C" __global__ __launch_bounds__(256) void vtb_xsplit_1(vtb::XSplitArgs a) { vtb::xsplit_body<1>(a); }
 
 // out = the n_split partials of each output, added in split order.  One wave
-// per token and row block, four rows per lane; partials of rows past m and
-// tokens past B were not written and are not read.
+// per token and row block, four rows per lane; a tile's rows past m were not
+// written: they are read with the others and not stored.
 extern "C" __global__ __launch_bounds__(256) void vtb_qgemm_reduce(vtb::QReduceArgs a) {
   const int lane = (int)threadIdx.x & 63, tok = 4 * (int)blockIdx.y + ((int)threadIdx.x >> 6), rb = (int)blockIdx.x;
   const int row = vtb::kQgRows * rb + 4 * lane;
@@ -704,20 +712,23 @@ extern "C" __global__ __launch_bounds__(256) void vtb_qgemm_reduce(vtb::QReduceA
   const float* p = a.part + ((size_t)tb * a.n_rb + rb) * tile + (size_t)(tok - tb * a.tile_tokens) * vtb::kQgRows + 4 * lane;
   float* o = a.out + (size_t)tok * a.m + row;
   const size_t step = (size_t)a.n_tb * a.n_rb * tile;
-  if (row + 4 <= a.m) {
-    float4 v = *reinterpret_cast<const float4*>(p);
-    for (int s = 1; s < a.n_split; ++s) {
-      const float4 u = *reinterpret_cast<const float4*>(p + s * step);
-      v = make_float4(v.x + u.x, v.y + u.y, v.z + u.z, v.w + u.w);
-    }
-    o[0] = v.x, o[1] = v.y, o[2] = v.z, o[3] = v.w;
-  } else {
-    for (int e = 0; row + e < a.m; ++e) {
-      float v = p[e];
-      for (int s = 1; s < a.n_split; ++s) v += p[s * step + e];
-      o[e] = v;
-    }
+  // Eight partials in flight; past the last one it is read again and not added.
+  // (One after the other, and the last rows of m % 4 on their own, 4096 x 4096
+  // with 33 tokens took 1.6 us more per call, 374 x 9216 with 40 12.)
+  float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  for (int s0 = 0; s0 < a.n_split; s0 += 8) {
+    float4 u[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      u[i] = *reinterpret_cast<const float4*>(p + (size_t)(s0 + i < a.n_split ? s0 + i : a.n_split - 1) * step);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (s0 + i < a.n_split) v = make_float4(v.x + u[i].x, v.y + u[i].y, v.z + u[i].z, v.w + u[i].w);
   }
+  const float r[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (row + e < a.m) o[e] = r[e];
 }
 
 // Two workgroups per CU (at most 256 registers per lane).

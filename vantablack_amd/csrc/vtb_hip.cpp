@@ -991,7 +991,7 @@ constexpr size_t kQgRows = 256;  // rows of a workgroup
 // in whole blocks of 256 columns, and vtb_qgemm_reduce adds the partials.
 // (Q4_K 1024 x 4096, 2048 tokens, 128 workgroups unsplit: 164 us with the former
 // 128 x 128 tiles, 72 split by four; 4096 x 4096, 33 tokens, 16 workgroups
-// unsplit: 151 and 23.)  Partials are tiles of 64 KiB, so n_split n_rb n_tb
+// unsplit: 151 and 21.)  Partials are tiles of 64 KiB, so n_split n_rb n_tb
 // <= 2 CUs bounds them whatever m and B.
 // Up to three weight matrices of one format over the same activations share
 // one pre-pass (the Q/K/V or gate/up projections of a prefill layer).
