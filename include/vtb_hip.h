@@ -400,8 +400,8 @@ int vtb_hip_kv_cache_shrink_to_fit(VtbHipKvCache *cache, size_t new_max_seq);
  * and gpuFinalStep (:515-520), one call.  x holds the token's embedding and is
  * left as the normalised residual stream, logits[vocab_size] the projection,
  * row pos of every layer's K/V slab ([n_layers][max_seq][n_kv_heads][head_dim]
- * of kv_dtype) the token's.  Norms and residual adds run inside the GEMVs next
- * to them; xb, xb2, q, k_cur, v_cur, attn_out, gate, up and ffn_out are scratch
+ * of kv_dtype) the token's.  Residual adds, and norms where that is
+ * faster, run inside the GEMVs next to them; xb, xb2, q, k_cur, v_cur, attn_out, gate, up and ffn_out are scratch
  * of the layer's sizes whose contents afterwards are unspecified.  Offsets are
  * bytes into weights; kinds 0 q8_0, 1 q4_k, 2 q5_k, 3 q6_k; activation 0 silu,
  * 1 gelu_approx. */

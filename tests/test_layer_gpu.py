@@ -243,7 +243,8 @@ class _Launches:
 # adds inside those that produce it, formats mixed in one launch) against the
 # single launches, over an f32 cache.  Widths: below one 2048-column slice
 # (four row waves per workgroup), exactly one with the rows for R = 4 and 2,
-# and two waves along k of which the second is partly past k; every format,
+# and two waves along k of which the second is partly past k (where one format
+# keeps the norm's own launch); every format,
 # gate and up of one format and of two, both activations.  Both sides are f32
 # and differ by the order of a few roundings of 2^-24 per activation (the
 # norm's scale before or after the dot), averaged over k: 1e-5 of the largest
@@ -254,6 +255,7 @@ class _Launches:
     (2048, 32, 4, 64, 5632, "silu", ("q4_k", "q4_k", "q6_k", "q4_k", "q4_k", "q4_k", "q6_k")),
     (2304, 18, 6, 128, 1280, "gelu_approx", ("q5_k", "q6_k", "q6_k", "q5_k", "q5_k", "q5_k", "q4_k")),
     (2304, 18, 3, 128, 768, "silu", ("q6_k", "q4_k", "q8_0", "q6_k", "q5_k", "q6_k", "q6_k")),
+    (2304, 18, 6, 128, 768, "silu", ("q4_k",) * 7),
 ])
 def test_token_step_matches_its_launches(ctx, dim, heads, n_kv, d, ffn, act, kinds):
     import vantablack_amd as vb

@@ -1845,7 +1845,7 @@ VTB_MATMUL_BATCHED_ENTRIES(q6_k, 3)
 // One token through every layer and the logits (gpuLayerStep per layer, then
 // gpuFinalStep), each rmsnorm inside the projections that read it and each
 // residual add inside the projection that produces it: five launches per
-// layer, whatever the formats.
+// layer, or seven (with `fuse` false and no formats mixed).
 extern "C" void vtb_hip_segment_token_step(VtbHipSeg* seg, const VtbHipTokenStep* t) {
   if (!seg) return;
   VtbHipCtx* ctx = seg->ctx;
@@ -1855,6 +1855,14 @@ extern "C" void vtb_hip_segment_token_step(VtbHipSeg* seg, const VtbHipTokenStep
                             ? 0 : t->pos - t->sliding_window + 1;
   const float inv_sqrt_hd = (float)(1.0 / std::sqrt((double)t->head_dim));
   const bool gelu = t->activation == 1;
+  // Beyond one 2048-column slice projections of one format keep the norm's own
+  // launch and the kernel of that format: the norm's loads and the registers of
+  // the widest format (131, half the waves of Q4_K's 76) cost more than the launch.
+  // 16 layers of 32/32 heads d128, ffn 11008, Q4_K: 867 us per token so with the
+  // residual adds apart, 891 with the norms inside; where formats differ, which
+  // takes a launch per projection otherwise, 1083 and 1006 (32/8 heads, ffn 14336,
+  // Q6_K V and down); 16/16 heads d64 (dim 1024) 490 and 384.
+  const bool fuse = t->dim <= 2048;
   struct Proj {
     size_t kind;
     VtbHipBuf* out;
@@ -1897,19 +1905,29 @@ extern "C" void vtb_hip_segment_token_step(VtbHipSeg* seg, const VtbHipTokenStep
     const VtbHipTokenLayer& L = t->layers[l];
     const Proj qkv[3] = {{L.kind_q, t->q, L.wq, t->dim}, {L.kind_k, t->k_cur, L.wk, kv_dim},
                          {L.kind_v, t->v_cur, L.wv, kv_dim}};
-    if (!norm_matmul(L.attn_norm, qkv, 3, 0)) {
+    const bool same = L.kind_q == L.kind_k && L.kind_k == L.kind_v && L.kind_q < (size_t)kNumQuant;
+    if ((same && !fuse) || !norm_matmul(L.attn_norm, qkv, 3, 0)) {
       vtb_hip_segment_rmsnorm(seg, t->xb, t->x, t->weights, L.attn_norm, t->dim, t->rms_eps);
-      for (const Proj& p : qkv) matmul(p, t->xb, t->dim);
+      if (same)
+        seg_note(seg, matmul3_entry(ctx, (int)L.kind_q, t->q, L.wq, t->dim, t->k_cur, L.wk, kv_dim, t->v_cur, L.wv, kv_dim,
+                                    t->weights, t->xb, t->dim));
+      else
+        for (const Proj& p : qkv) matmul(p, t->xb, t->dim);
     }
     const size_t off = l * t->max_seq * row_bytes + wstart * row_bytes;
     vtb_hip_segment_attn_decode_rope_append(seg, t->attn_out, t->q, t->kv_k, off, t->kv_v, off, t->k_cur, t->v_cur,
                                             t->n_heads, t->n_kv_heads, t->head_dim, t->pos + 1 - wstart, inv_sqrt_hd,
                                             t->kv_dtype, t->pos, t->rope_base, t->rope_half);
     matmul_add(L.kind_o, t->xb2, L.wo, t->attn_out, t->dim);
-    const bool gated = L.kind_gate == L.kind_up;  // gate takes the pair's output
     const Proj ffn[2] = {{L.kind_gate, t->gate, L.wgate, t->ffn_dim}, {L.kind_up, t->up, L.wup, t->ffn_dim}};
-    if (!gated || !norm_matmul(L.ffn_norm, ffn, 2, gelu ? 2 : 1)) {
-      if (gated || !norm_matmul(L.ffn_norm, ffn, 2, 0)) {
+    if (L.kind_gate == L.kind_up && L.kind_gate < (size_t)kNumQuant) {  // gate takes the pair's output
+      if (!fuse || !norm_matmul(L.ffn_norm, ffn, 2, gelu ? 2 : 1)) {
+        vtb_hip_segment_rmsnorm(seg, t->xb, t->x, t->weights, L.ffn_norm, t->dim, t->rms_eps);
+        seg_note(seg, matmul_gated_entry(ctx, (int)L.kind_gate, t->gate, t->weights, L.wgate, L.wup, t->xb, t->ffn_dim,
+                                         t->dim, t->activation));
+      }
+    } else {
+      if (!norm_matmul(L.ffn_norm, ffn, 2, 0)) {
         vtb_hip_segment_rmsnorm(seg, t->xb, t->x, t->weights, L.ffn_norm, t->dim, t->rms_eps);
         for (const Proj& p : ffn) matmul(p, t->xb, t->dim);
       }

@@ -18,9 +18,10 @@ each residual add fused into the rmsnorm that follows it
 launch (vtb_hip_segment_matmul3_<kind>) and the gate/up GEMVs with the
 activation in one launch (vtb_hip_segment_matmul_gated_<kind>) when the
 projections share a format: 7 launches per layer instead of 13, the same
-arithmetic per output.  A hip.Segment encodes it in one native call of 5
-launches per layer (vtb_hip_segment_token_step): each norm inside the
-projections that read it, each residual add inside the one that produces it.
+arithmetic per output.  A hip.Segment encodes it in one native call
+(vtb_hip_segment_token_step) with each residual add inside the projection
+that produces it and, up to dim 2048 or where formats are mixed, each norm
+inside the projections that read it: 5 launches per layer.
 
 The sliding window is the reference's caller-side offset shift
 (forward.zig:470-480): the K/V base moves to the window's first row and the
