@@ -424,8 +424,8 @@ void vtb_hip_segment_token_step(VtbHipSeg *seg, const VtbHipTokenStep *step);
  * score rows for max_seq once, before the first forward.  Grows, once, every
  * buffer the context otherwise grows on demand (which drains the stream and
  * calls hipMalloc inside the call that needs it): the split-K decode
- * workspace and counters for one query (and, on f32 caches, whose prefill
- * runs the decode kernel, up to max_batch queries) over up to c->max_seq
+ * workspace and counters for one query (and, on f32 caches, whose prefill of
+ * few queries runs the decode kernel, up to max_batch queries) over up to c->max_seq
  * keys or the window; the prefill conversion scratch for a c->max_seq-key
  * context (f16/bf16 caches, max_batch > 0); the batched-matmul activation
  * scratch for max_batch tokens of width max_matmul_k (0: none); for both of
